@@ -34,121 +34,340 @@ DF_DEVICE float readlane(float v, int lane) {
 //
 // The weight is in the library's device tiling (df_int4_repack). A 1 KB block is 16 columns x
 // one 128-group, and lane L of a 64-lane read owns its bytes [16 L, 16 L + 16): four words of
-// column L % 16. Word i holds k = 32 (L / 16) + 8 i + e, e < 8, with element e at bit
-// 4 (e / 2), plus 16 when e is odd. That is exactly the B operand of
-// v_mfma_f32_16x16x32_bf16 number i, whose A operand is then x[row][32 (L / 16) + 8 i ..+8].
-// A workgroup computes a 128 x 128 tile; wave w owns all 128 rows and column tiles 2w, 2w + 1
-// (8 x 2 products). Per 128-group:
-// - only the x rows go through LDS, double-buffered (one barrier per group): the next
-//   group's rows are stored from registers while this group's products run;
-// - each wave loads its two weight blocks straight into registers a group ahead, in the
-//   MFMA B layout, and dequantises them there with int4_block.h's exact dequant (19 VALU per
-//   8 weights), so every weight is dequantised once and never staged.
-// The products, and each output's order of summation, are those of a staged-B design.
+// column L % 16. Word i holds k = 32 (L / 16) + 8 i + e, e < 8, which is exactly the B operand
+// of v_mfma_f32_16x16x32_bf16 number i, whose A operand is then x[row][32 (L / 16) + 8 i ..+8]
+// (the decode GEMV's products).
+//
+// A workgroup computes tiles of RB row blocks of 32 x WN * CP column pairs (two 16-column tiles,
+// 32 columns) on v_mfma_f32_32x32x16_bf16. Step n of a group takes word n % 4 of slots
+// 2 (n / 4) and 2 (n / 4) + 1 (lanes 0..31 and 32..63): B operand as loaded, and
+// x[row][128 g + 32 slot + 8 (n % 4) ..+8] as A. Its 2 WN waves are two sets: set s sums the
+// groups g = s, s + 2, .. of the tile in order, and the result is set 0's sum plus set 1's, in
+// every launch shape. So an output's bits do not depend on M, N or the shape chosen (a prompt
+// filled in chunks equals one pass).
+// - A stage is one group of each set. x rows go to LDS by global_load_lds (no registers), NBUF
+//   stages in a ring, one barrier per stage; a row's 16-byte chunk c sits in slot
+//   c ^ (row % 16), so the rows of an A operand read spread over the banks.
+// - WREG shapes (long prompts): each wave loads its blocks and scales of the next stage into
+//   registers. Otherwise blocks and scales go through the LDS ring too, NBUF - 1 stages ahead:
+//   the narrow shapes' stages are shorter than a memory round trip.
+// - Every wave dequantises its own blocks (17 VALU per 8 weights), the next step's during the
+//   products of this one; A operands are read a step (narrow shapes: more) ahead.
+// - WREG workgroups are persistent, one per CU: the next tile's first stage loads while the
+//   sums of this one meet in LDS, 32 rows at a time, and leave as 16-byte stores.
+// What bounds it: 128 x 256 tiles take 5950 cycles a stage for 4096 of products and 2200 of
+// dequant (MFMA and VALU of a SIMD's two waves share its issue), and with every CU busy the
+// clock falls to 1.73 GHz under the power limit (2.4 with 10 CUs busy). Before (128 x 128 tiles,
+// each wave all 128 rows x 32 columns on 16 x 16 x 32 products, x through registers, one
+// group's weights ahead) -> now, us: gate|up 4096 x 2560 x 18432 505 -> 360 (1074 TFLOP/s; a
+// plain bf16 library product of that shape 368), down 4096 x 9216 x 2560 301 -> 187, at 100
+// rows 38.6 -> 22.9 and 115 -> 26.5. Tried and not kept: 16 x 16 x 32 products (same stage time,
+// twice the operand reads), forcing products and VALU to alternate one by one (1 to 3 %
+// slower), wave priorities (no change), 320-column tiles (spill).
 
-constexpr int kGmBM = 128;
-constexpr int kGmTiles = 8;           // 16-column tiles per workgroup (128 columns)
-constexpr int kGmXPitch = 128 + 8;    // bf16 per staged x row (16-byte pad)
+constexpr int kGmMaxLds = 160 * 1024;
+constexpr int kCUs = 256;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+DF_DEVICE f32x16 mfma32(const uint4& a, const uint4& b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(df_bf16x8, a), __builtin_bit_cast(df_bf16x8, b),
+                                                 c, 0, 0, 0);
+}
 
-template <int EPI>
-__global__ __launch_bounds__(256, 2) void int4_gemm_kernel(DfInt4GemmArgs p) {
-  __shared__ __align__(16) uint16_t xs[2][kGmBM * kGmXPitch];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * kGmBM, t0 = blockIdx.x * kGmTiles + 2 * wave;
-  const int G = p.K / 128, ntiles = p.N / 16;
-  df_f32x4 acc[8][2];
-#pragma unroll
-  for (int rb = 0; rb < 8; ++rb)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[rb][j] = df_f32x4{0.f, 0.f, 0.f, 0.f};
+struct GemmGeom {
+  int mblocks, nblocks;  // workgroups along M and N
+  int flags;             // kGmVecOut, kGmScale4
+};
+constexpr int kGmVecOut = 1;  // out and ldo allow 16-byte stores
+constexpr int kGmScale4 = 2;  // s is 4-byte aligned (the scale DMA moves dwords)
 
-  uint4 xr[8], wr[2];
-  uint16_t sr[2];
-  auto load_x = [&](int g) {
+template <int RB, int CP, int WN, int NBUF, bool WREG>
+struct GemmShape {
+  static constexpr int BM = 32 * RB, BN = 32 * CP * WN, kThreads = 128 * WN;
+  static constexpr int kTiles = 2 * CP * WN;             // 16-column tiles
+  static constexpr int kRegion = BM * 256;               // one group of the x rows
+  static constexpr int kXBytes = 2 * kRegion;            // both sets' groups
+  static constexpr int kXOps = BM / (4 * WN);            // x DMAs per wave and stage
+  static constexpr int kWBytes = WREG ? 0 : kTiles * 2048;
+  static constexpr int kSOps = (kTiles + 3) / 4;        // scale DMAs (4 tiles each) per stage
+  static constexpr int kSBytes = WREG ? 0 : kSOps * 256;
+  static constexpr int kStage = kXBytes + kWBytes + kSBytes;
+  static constexpr int kOps = kXOps + (WREG ? 0 : 2 * CP + 1);  // DMAs per wave and stage
+  static constexpr int kPitch = BN + 4;                  // fp32 row pitch of the epilogue
+  static constexpr int kEpi = 2 * 32 * kPitch * 4;
+  // WREG: the sums meet past the first buffer, which already receives the next tile's rows
+  static constexpr int kEpiOff = WREG ? kStage : 0;
+  static constexpr int kLds = NBUF * kStage > kEpiOff + kEpi ? NBUF * kStage : kEpiOff + kEpi;
+  static_assert(BM % (8 * WN) == 0 && kLds <= kGmMaxLds && (!WREG || NBUF == 2), "shape");
+};
+
+// 16 (4) bytes per lane from global memory to LDS at lds_base + 16 (4) * lane. Inline asm, so
+// that the compiler does not wait for all of them before any LDS read; the kernel waits itself.
+DF_DEVICE void dma16(const void* gaddr, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gaddr), "s"(lds_base)
+               : "memory", "m0");
+}
+DF_DEVICE void dma4(const void* gaddr, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(gaddr), "s"(lds_base)
+               : "memory", "m0");
+}
+// x / (1 + e^-x) from the hardware's exp2 and reciprocal instead of expf and an IEEE division:
+// 5 VALU instead of about 40. Relative error about 6e-8 (2 + |x|), against the 2e-3 of the bf16
+// rounding that follows; the expf form took 6 us of a 128 x 256 tile's 40.
+DF_DEVICE float silu_fast(float x) {
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * x));
+}
+template <int N>
+DF_DEVICE void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+typedef __attribute__((address_space(3))) unsigned char lds_byte;
+DF_DEVICE uint32_t lds_offset(const void* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const lds_byte*)p));
+}
+
+template <int EPI, int RB, int CP, int WN, int NBUF, bool WREG>
+__global__ __launch_bounds__(128 * WN, 1) void int4_gemm_kernel(DfInt4GemmArgs p, GemmGeom geo) {
+  using SH = GemmShape<RB, CP, WN, NBUF, WREG>;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kset = wave / WN, wn = wave % WN;
+  const int G = p.K / 128, ntiles = p.N / 16, stages = G / 2;
+
+  // Workgroups go to XCDs round-robin by index. Each XCD takes a contiguous run of the tile
+  // order, which walks 8 row blocks down before the next column block, so that the workgroups
+  // of an XCD share x rows and weight blocks in its L2. WREG workgroups are one per CU and
+  // walk their XCD's run; the others have one tile.
+  const int total = geo.mblocks * geo.nblocks, xcd = blockIdx.x & 7;
+  const int run = (total >> 3) * xcd + min(xcd, total & 7), run_end = run + (total >> 3) + (xcd < (total & 7) ? 1 : 0);
+  const int stride = static_cast<int>(gridDim.x) < total ? static_cast<int>(gridDim.x) >> 3 : total;
+  int tile = run + (blockIdx.x >> 3);
+  if (tile >= run_end) return;
+
+  // x: this thread's 16-byte chunks of a stage. Chunk i of thread tid lands at byte
+  // (i * threads + tid) * 16 of the stage: row (i * 8 WN + tid / 16) % BM of a set's group,
+  // slot tid % 16. Rows past M read row M - 1 (their results are not stored).
+  const unsigned char* xp[SH::kXOps / 2];
+  int m0, tile0, t0;
+  auto start_tile = [&](int t) {
+    const int per = 8 * geo.nblocks, grp = t / per, in = t - grp * per;
+    const int rows = min(8, geo.mblocks - grp * 8);
+    const int nb = in / rows, mb = grp * 8 + (in - nb * rows);
+    m0 = mb * SH::BM;
+    tile0 = nb * SH::kTiles;
+    t0 = tile0 + wn * 2 * CP;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {  // 128 rows x 16 chunks of 16 bytes
-      const int ch = tid + 256 * i, r = ch >> 4, cc = ch & 15;
-      xr[i] = m0 + r < p.M ? *reinterpret_cast<const uint4*>(p.x + (size_t)(m0 + r) * p.ldx + g * 128 + cc * 8)
-                           : make_uint4(0u, 0u, 0u, 0u);
+    for (int i = 0; i < SH::kXOps / 2; ++i) {
+      const int r = i * 8 * WN + (tid >> 4);
+      const int c = (tid & 15) ^ (r & 15);
+      xp[i] = reinterpret_cast<const unsigned char*>(p.x + (size_t)min(m0 + r, p.M - 1) * p.ldx) + c * 16;
     }
   };
-  auto store_x = [&](int buf) {
+  start_tile(tile);
+  const uint32_t lds0 = lds_offset(smem) + wave * 1024;
+  auto issue_x = [&](int st, int buf) {
+    const uint32_t base = lds0 + buf * SH::kStage;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int ch = tid + 256 * i, r = ch >> 4, cc = ch & 15;
-      *reinterpret_cast<uint4*>(&xs[buf][r * kGmXPitch + cc * 8]) = xr[i];
+    for (int i = 0; i < SH::kXOps; ++i) {
+      const int set = i / (SH::kXOps / 2);
+      dma16(xp[i % (SH::kXOps / 2)] + (size_t)st * 512 + set * 256, base + i * (SH::kThreads * 16));
     }
   };
-  auto load_w = [&](int g) {  // this wave's two blocks of group g (zeros past N)
+  // Blocks through LDS: wave's DMA j moves block wave * 2 CP + j of [tile][group of the stage];
+  // a tile's two groups are contiguous in memory. Scales: [tile][group][16], 4 tiles per DMA.
+  auto issue_w = [&](int st, int buf) {
+    const uint32_t base = lds_offset(smem) + buf * SH::kStage + SH::kXBytes;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      wr[j] = make_uint4(0x88888888u, 0x88888888u, 0x88888888u, 0x88888888u);
-      sr[j] = 0;
-      if (t0 + j < ntiles) {
-        const size_t blk = (size_t)(t0 + j) * G + g;
-        wr[j] = *reinterpret_cast<const uint4*>(p.w + blk * 1024 + lane * 16);
-        sr[j] = p.s[blk * 16 + (lane & 15)];
+    for (int j = 0; j < 2 * CP; ++j) {
+      const int blk = wave * 2 * CP + j, t = min(tile0 + (blk >> 1), ntiles - 1);
+      dma16(p.w + ((size_t)t * G + 2 * st + (blk & 1)) * 1024 + lane * 16, base + blk * 1024);
+    }
+    const int op = wave % SH::kSOps, t = min(tile0 + op * 4 + (lane >> 4), ntiles - 1);
+    const uint16_t* src = p.s + ((size_t)t * G + 2 * st) * 16 + (lane & 15) * 2;
+    const uint32_t dst = base + SH::kWBytes + op * 256;
+    if (geo.flags & kGmScale4) {
+      dma4(src, dst);
+    } else {
+      const uint32_t v = src[0] | (static_cast<uint32_t>(src[1]) << 16);
+      *reinterpret_cast<uint32_t*>(smem + (dst - lds_offset(smem)) + lane * 4) = v;
+    }
+  };
+
+  // Column lane % 32 of pair cp is column lane % 16 of tile 2 cp + (lane / 16) % 2; the lane's
+  // half (lane / 32) holds slots h and 2 + h of its block, 16 bytes each.
+  const int half = lane >> 5, odd = (lane >> 4) & 1, lcol = lane & 15, lrow = lane & 31;
+  const uint32_t woff = half * 256 + lcol * 16;
+  uint4 wq[CP][2];
+  uint32_t sq[CP];
+  auto load_w = [&](int st) {
+    const int g = 2 * st + kset;
+#pragma unroll
+    for (int c = 0; c < CP; ++c) {
+      const size_t blk = (size_t)min(t0 + 2 * c + odd, ntiles - 1) * G + g;
+      wq[c][0] = load16(p.w + blk * 1024 + woff);
+      wq[c][1] = load16(p.w + blk * 1024 + 512 + woff);
+      sq[c] = p.s[blk * 16 + lcol];
+    }
+  };
+
+  f32x16 acc[RB][CP];
+  const DqK K = dq_consts();
+  uint4 wr[CP][2];      // this set's group of the stage: the wave's blocks
+  GroupScale gs[CP];
+  // Operands of step n: a[n % (kAhead + 1)], read kAhead steps before, and b[n & 1].
+  constexpr int kAhead = RB >= 3 ? 1 : RB == 2 ? 3 : 7;
+  uint4 a[kAhead + 1][RB], b[2][CP];
+  auto word = [&](int c, int n) {
+    const uint4 v = wr[c][n >> 2];
+    return (n & 3) == 0 ? v.x : (n & 3) == 1 ? v.y : (n & 3) == 2 ? v.z : v.w;
+  };
+  // takes over the blocks loaded by load_w: the compiler waits for them here and not later, when
+  // its wait would include DMAs that it does not count
+  auto take_w = [&](int c) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      asm volatile("" : "+v"(wq[c][h].x), "+v"(wq[c][h].y), "+v"(wq[c][h].z), "+v"(wq[c][h].w));
+      wr[c][h] = wq[c][h];
+    }
+    asm volatile("" : "+v"(sq[c]));
+    gs[c] = group_scale(static_cast<uint16_t>(sq[c]));
+  };
+  auto first_stages = [&]() {
+    if constexpr (WREG) {
+      load_w(0);
+      issue_x(0, 0);
+    } else {
+#pragma unroll
+      for (int n = 0; n < NBUF - 1; ++n)
+        if (n < stages) {
+          issue_x(n, n);
+          issue_w(n, n);
+        }
+    }
+  };
+  first_stages();
+  for (;;) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int c = 0; c < CP; ++c)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[rb][c][e] = 0.f;
+    if constexpr (WREG) {
+#pragma unroll
+      for (int c = 0; c < CP; ++c) {
+        take_w(c);
+        b[0][c] = dequant8(word(c, 0), gs[c], K);
       }
     }
-  };
-  load_x(0);
-  load_w(0);
-  store_x(0);
-  if (G > 1) load_x(1);
-  const DqK K = dq_consts();
-  for (int g = 0; g < G; ++g) {
-    // xs[g & 1] is complete, and every wave is done with xs[(g + 1) & 1] (group g - 1)
-    __syncthreads();
-    uint4 b[2][4];
+    int buf = 0;
+    for (int st = 0; st < stages; ++st) {
+      // This wave's part of stage st is in LDS: later stages' DMAs may still be in flight.
+      if (st + NBUF - 2 < stages)
+        wait_vm<(NBUF - 2) * SH::kOps>();
+      else
+        wait_vm<0>();
+      // every wave's part is, and every wave is done with the buffer that is filled next
+      __syncthreads();
+      if (st + NBUF - 1 < stages) {
+        const int next = buf == 0 ? NBUF - 1 : buf - 1;
+        if constexpr (WREG) load_w(st + 1);
+        issue_x(st + NBUF - 1, next);
+        if constexpr (!WREG) issue_w(st + NBUF - 1, next);
+      }
+      const unsigned char* sb = smem + buf * SH::kStage;
+      const unsigned char* xs = sb + kset * SH::kRegion + lrow * 256;
+      auto read_a = [&](int n) {
+        const uint32_t at = ((8 * (n >> 2) + 4 * half + (n & 3)) ^ lcol) << 4;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const GroupScale gs = group_scale(sr[j]);  // the exact bf16((n - 8) * scale) of the per-op GEMV
-      b[j][0] = dequant8(wr[j].x, gs, K);
-      b[j][1] = dequant8(wr[j].y, gs, K);
-      b[j][2] = dequant8(wr[j].z, gs, K);
-      b[j][3] = dequant8(wr[j].w, gs, K);
+        for (int rb = 0; rb < RB; ++rb) a[n % (kAhead + 1)][rb] = *reinterpret_cast<const uint4*>(xs + rb * 8192 + at);
+      };
+#pragma unroll
+      for (int n = 0; n < kAhead; ++n) read_a(n);
+      if constexpr (!WREG) {
+#pragma unroll
+        for (int c = 0; c < CP; ++c) {
+          const int blk = 2 * (wn * 2 * CP + 2 * c + odd) + kset;
+          const unsigned char* w = sb + SH::kXBytes + blk * 1024 + woff;
+          wr[c][0] = *reinterpret_cast<const uint4*>(w);
+          wr[c][1] = *reinterpret_cast<const uint4*>(w + 512);
+          gs[c] = group_scale(*reinterpret_cast<const uint16_t*>(sb + SH::kXBytes + SH::kWBytes + blk * 32 + lcol * 2));
+          b[0][c] = dequant8(word(c, 0), gs[c], K);
+        }
+      }
+      // 8 steps of 16 k: a step's A operands are read kAhead steps before and its B operands
+      // dequantised between the products of the step before.
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < 8; ++n) {
+        if (n + kAhead < 8) read_a(n + kAhead);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+          for (int c = 0; c < CP; ++c) acc[rb][c] = mfma32(a[n % (kAhead + 1)][rb], b[n & 1][c], acc[rb][c]);
+#pragma unroll
+        for (int c = 0; c < CP; ++c) {
+          if (n < 7) {
+            b[(n + 1) & 1][c] = dequant8(word(c, n + 1), gs[c], K);
+          } else if (WREG) {
+            take_w(c);
+            b[0][c] = dequant8(word(c, 0), gs[c], K);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      buf = buf + 1 == NBUF ? 0 : buf + 1;
     }
-    if (g + 1 < G) {
-      store_x((g + 1) & 1);
-      load_w(g + 1);
-    }
-    if (g + 2 < G) load_x(g + 2);
-    const uint16_t* xb = xs[g & 1];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      uint4 a[8];
-#pragma unroll
-      for (int rb = 0; rb < 8; ++rb)
-        a[rb] = *reinterpret_cast<const uint4*>(&xb[(rb * 16 + (lane & 15)) * kGmXPitch + (lane >> 4) * 32 + i * 8]);
-#pragma unroll
-      for (int rb = 0; rb < 8; ++rb)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[rb][j] = mfma(a[rb], b[j][i], acc[rb][j]);
-    }
-  }
 
-  // lane holds D[4 (lane / 16) + r][lane % 16] of each 16 x 16 product
-  const int col_in = lane & 15;
+    // The sets' sums, 32 rows at a time: lane holds D[(e % 4) + 8 (e / 4) + 4 (lane / 32)][lane % 32]
+    // of each 32 x 32 product; 8 columns of a row leave together.
+    const int em0 = m0, etile0 = tile0;
+    __syncthreads();
+    tile += stride;
+    if (tile < run_end) {  // the next tile's first stage arrives during the stores
+      start_tile(tile);
+      first_stages();
+    }
+    float* ep = reinterpret_cast<float*>(smem + SH::kEpiOff);
+    constexpr int kOutCols = EPI == DF_EPI_SWIGLU ? SH::BN / 2 : SH::BN;
+    const int out_col0 = EPI == DF_EPI_SWIGLU ? etile0 * 8 : etile0 * 16;
+    const int out_n = EPI == DF_EPI_SWIGLU ? p.N / 2 : p.N;
 #pragma unroll
-  for (int rb = 0; rb < 8; ++rb) {
+    for (int h = 0; h < RB; ++h) {
+      if (h > 0) __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = m0 + rb * 16 + (lane >> 4) * 4 + r;
-      if (row >= p.M) continue;
-      if (EPI == DF_EPI_SWIGLU) {
-        // tiles alternate gate, up: this wave's pair (2w, 2w + 1);
-        // bf16(bf16(silu(bf16(g))) * bf16(u)) (reference.py:692-693)
-        if (t0 >= ntiles) continue;
-        const float gv = round_bf(acc[rb][0][r]), uv = round_bf(acc[rb][1][r]);
-        p.out[(size_t)row * p.ldo + (t0 / 2) * 16 + col_in] = f2bf(round_bf(silu(gv)) * uv);
-      } else {
+      for (int c = 0; c < CP; ++c)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          if (t0 + j >= ntiles) continue;
-          p.out[(size_t)row * p.ldo + (t0 + j) * 16 + col_in] = f2bf(acc[rb][j][r]);
+        for (int e = 0; e < 16; ++e)
+          ep[(kset * 32 + (e & 3) + 8 * (e >> 2) + 4 * half) * SH::kPitch + (wn * CP + c) * 32 + lrow] = acc[h][c][e];
+      __syncthreads();
+      for (int u = tid; u < 32 * kOutCols / 8; u += SH::kThreads) {
+        const int row = u / (kOutCols / 8), c = (u - row * (kOutCols / 8)) * 8;
+        const int m = em0 + h * 32 + row, col = out_col0 + c;
+        if (m >= p.M || col >= out_n) continue;
+        float y[8];
+        if constexpr (EPI == DF_EPI_SWIGLU) {
+          // tiles alternate gate, up: bf16(bf16(silu(bf16(g))) * bf16(u)) (reference.py:692-693)
+          const float* g = ep + row * SH::kPitch + (c / 16) * 32 + (c & 15);
+          const float* g1 = g + 32 * SH::kPitch;
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            y[e] = round_bf(silu_fast(round_bf(g[e] + g1[e]))) * round_bf(g[16 + e] + g1[16 + e]);
+        } else {
+          const float* g = ep + row * SH::kPitch + c;
+          const float* g1 = g + 32 * SH::kPitch;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[e] = g[e] + g1[e];
+        }
+        uint16_t* dst = p.out + (size_t)m * p.ldo + col;
+        if (geo.flags & kGmVecOut) {
+          *reinterpret_cast<uint4*>(dst) = make_uint4(pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]),
+                                                      pack_bf16(y[4], y[5]), pack_bf16(y[6], y[7]));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) dst[e] = f2bf(y[e]);
         }
       }
     }
+    if (tile >= run_end) break;
   }
 }
 
@@ -847,6 +1066,62 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(DfAttnPrefillArgs 
 using namespace df;
 using namespace df::pf;
 
+template <int EPI, int RB, int CP, int WN, int NBUF, bool WREG>
+static hipError_t launch_gemm_shape(const DfInt4GemmArgs& a, hipStream_t stream) {
+  using SH = GemmShape<RB, CP, WN, NBUF, WREG>;
+  GemmGeom geo;
+  geo.mblocks = (a.M + SH::BM - 1) / SH::BM;
+  geo.nblocks = (a.N / 16 + SH::kTiles - 1) / SH::kTiles;
+  geo.flags = (((reinterpret_cast<uintptr_t>(a.out) & 15) == 0 && a.ldo % 8 == 0) ? kGmVecOut : 0) |
+              ((reinterpret_cast<uintptr_t>(a.s) & 3) == 0 ? kGmScale4 : 0);
+  const long total = (long)geo.mblocks * geo.nblocks;
+  if (total > 0x7FFFFFFF) return hipErrorInvalidValue;
+  const unsigned grid = WREG && total > kCUs ? kCUs : (unsigned)total;
+  hipLaunchKernelGGL((int4_gemm_kernel<EPI, RB, CP, WN, NBUF, WREG>), dim3(grid), dim3(SH::kThreads), SH::kLds, stream,
+                     a, geo);
+  return hipGetLastError();
+}
+
+// The shapes, and the cost of one workgroup in each: start and epilogue, and a stage (ns). Fitted
+// to 60 measured (M, K, N): the four projections of the model at 17 .. 8192 rows. A launch
+// takes as many rounds of one workgroup per CU as it has tiles, so the shape taken is the one
+// with the least rounds * (start + stages * stage); over the 60 it was the fastest of the
+// seven but for 0.04 %. Wide ones serve long prompts (2560 x 18432 at 4096 rows: 9 full rounds of
+// 128 x 256, 360 us against 410 with 128 x 128), 96 rows where they pack better (9216 x 2560 at
+// 4096 rows: 187 us against 222), narrow ones reach more CUs with a short prompt (9216 x 2560
+// at 100 rows: 26.5 us with 32 x 64 against 96 with 128 x 256).
+struct GemmCost {
+  int bm, bn, start, stage;
+};
+constexpr GemmCost kGemmCosts[] = {{128, 256, 9000, 2650}, {128, 128, 5000, 1750}, {96, 256, 7000, 2250},
+                                   {96, 128, 4000, 1350},  {64, 128, 3200, 1100},  {64, 64, 2000, 880},
+                                   {32, 64, 1500, 710}};
+
+static int gemm_plan(int M, int K, int N) {
+  int best = 0;
+  double best_cost = 0;
+  for (int i = 0; i < static_cast<int>(sizeof(kGemmCosts) / sizeof(kGemmCosts[0])); ++i) {
+    const GemmCost& c = kGemmCosts[i];
+    const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    const double cost = (double)((tiles + kCUs - 1) / kCUs) * (c.start + (double)c.stage * (K / 256));
+    if (i == 0 || cost < best_cost) best = i, best_cost = cost;
+  }
+  return best;
+}
+
+template <int EPI>
+static hipError_t launch_gemm(const DfInt4GemmArgs& a, int shape, hipStream_t stream) {
+  switch (shape) {
+    case 0: return launch_gemm_shape<EPI, 4, 2, 4, 2, true>(a, stream);
+    case 1: return launch_gemm_shape<EPI, 4, 1, 4, 2, true>(a, stream);
+    case 2: return launch_gemm_shape<EPI, 3, 2, 4, 2, true>(a, stream);
+    case 3: return launch_gemm_shape<EPI, 3, 1, 4, 2, true>(a, stream);
+    case 4: return launch_gemm_shape<EPI, 2, 1, 4, 2, true>(a, stream);
+    case 5: return launch_gemm_shape<EPI, 2, 1, 2, 3, false>(a, stream);
+    default: return launch_gemm_shape<EPI, 1, 1, 2, 4, false>(a, stream);
+  }
+}
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 extern "C" {
@@ -859,15 +1134,13 @@ int df_int4_gemm(const DfInt4GemmArgs* a, hipStream_t stream) {
   const int out_cols = a->epilogue == DF_EPI_SWIGLU ? a->N / 2 : a->N;
   if (a->ldx < a->K || a->ldx % 8 || a->ldo < out_cols || !aligned16(a->x) || !aligned16(a->w))
     return DF_BAD_ARGUMENT;
-  const dim3 grid((a->N / 16 + kGmTiles - 1) / kGmTiles, (a->M + kGmBM - 1) / kGmBM);
-  if (grid.y > 65535) return DF_BAD_ARGUMENT;
-  if (a->epilogue == DF_EPI_SWIGLU)
-    hipLaunchKernelGGL(int4_gemm_kernel<DF_EPI_SWIGLU>, grid, dim3(256), 0, stream, *a);
-  else
-    hipLaunchKernelGGL(int4_gemm_kernel<DF_EPI_STORE>, grid, dim3(256), 0, stream, *a);
-  DF_RETURN_LAUNCH_STATUS();
+  // row blocks of the smallest shape fit the grid
+  if ((a->M + 127) / 128 > 65535) return DF_BAD_ARGUMENT;
+  const int shape = gemm_plan(a->M, a->K, a->N);
+  const hipError_t e = a->epilogue == DF_EPI_SWIGLU ? launch_gemm<DF_EPI_SWIGLU>(*a, shape, stream)
+                                                    : launch_gemm<DF_EPI_STORE>(*a, shape, stream);
+  return e == hipSuccess ? DF_OK : DF_LAUNCH_FAILED;
 }
-
 int df_causal_conv_prefill(const uint16_t* x, int ldx, int tokens, int channels, const uint16_t* weight,
                            uint16_t* ring, int pos0, uint16_t* out, int ldo, hipStream_t stream) {
   if (!x || !weight || !ring || !out || tokens < 1 || channels < 1 || ldx < channels || ldo < channels || pos0 < 0 ||

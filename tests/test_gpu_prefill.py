@@ -76,6 +76,40 @@ def test_int4_gemm_strided_rows_and_swiglu_epilogue():
     close(got, want, what="gate|up + SwiGLU", flip_frac=2e-3)
 
 
+# (M, K, N) that take each launch shape (128 x 256, 128 x 128, 96 x 256, 96 x 128, 64 x 128, 64 x 64,
+# 32 x 64) with a partial last row block, a partial last column block and one or more rounds
+@pytest.mark.parametrize("m,k,n,epilogue", [
+    (700, 512, 8208, N.EPI_STORE), (300, 512, 8208, N.EPI_STORE), (641, 512, 6176, N.EPI_SWIGLU),
+    (161, 512, 12304, N.EPI_STORE), (97, 512, 8208, N.EPI_STORE), (33, 768, 8224, N.EPI_SWIGLU),
+    (31, 768, 1040, N.EPI_STORE), (2100, 256, 4128, N.EPI_SWIGLU)])
+def test_int4_gemm_rows_do_not_depend_on_the_launch_shape(m, k, n, epilogue):
+    """Each shape against the expression on its first, last and some middle rows, and bit for
+    bit against the same rows as products of their own (other launch shapes); then with an output
+    and scales that allow neither 16-byte stores nor 4-byte loads."""
+    print(f"gemm shapes {m}x{k}x{n} epilogue {epilogue}", flush=True)
+    gen = torch.Generator().manual_seed(m + n)
+    w = synth.draw_int4(gen, k, -(-n // 64) * 64)
+    x = torch.randn((m, k), generator=gen).to(torch.bfloat16)
+    xd, whole = x.to(DEV), repack(w)
+    tiles = n // 16 * (k // 128)  # the first n columns are the first n / 16 tiles
+    weight = ops.Int4Weight(whole.w[:tiles * 1024], whole.s[:tiles * 16], k, n)
+    got = int4_gemm(xd, weight, epilogue=epilogue)
+    rows = torch.tensor(sorted({0, 1, min(31, m - 1), m // 2, m - 2, m - 1}))
+    want = dequant_gemv(x[rows], w.packed, w.scale, 128)[:, :n]
+    if epilogue == N.EPI_SWIGLU:  # 16-column gate / up tiles alternate
+        gu = want.reshape(len(rows), n // 32, 2, 16)
+        want = (F.silu(gu[:, :, 0]) * gu[:, :, 1]).reshape(len(rows), n // 2)
+    close(got[rows.to(DEV)], want, what=f"gemm {m}x{k}x{n}", flip_frac=2e-3)
+    for r0, r1 in ((0, 1), (0, min(m, 40)), (m // 2, m), (m - 1, m)):
+        assert torch.equal(int4_gemm(xd[r0:r1], weight, epilogue=epilogue), got[r0:r1]), (r0, r1)
+    cols = got.shape[1]
+    odd = torch.zeros((m, cols + 3), dtype=torch.bfloat16, device=DEV)[:, 1:1 + cols]
+    scales = torch.zeros(weight.s.numel() + 1, dtype=torch.bfloat16, device=DEV)[1:]
+    scales.copy_(weight.s)
+    int4_gemm(xd, ops.Int4Weight(weight.w, scales, k, n), epilogue=epilogue, out=odd)
+    assert torch.equal(odd, got)
+
+
 def test_int4_gemm_rejects_bad_shapes():
     gen = torch.Generator().manual_seed(4)
     w = repack(synth.draw_int4(gen, 256, 64))
