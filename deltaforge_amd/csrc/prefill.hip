@@ -116,6 +116,11 @@ DF_DEVICE void dma4(const void* gaddr, uint32_t lds_base) {
 DF_DEVICE float silu_fast(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * x));
 }
+// The same with the global address as a uniform base plus the lane's offset.
+DF_DEVICE void dma16s(const void* base, uint32_t offset, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_base)
+               : "memory", "m0");
+}
 template <int N>
 DF_DEVICE void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
@@ -875,187 +880,322 @@ __global__ __launch_bounds__(256) void qk_rows_kernel(DfQkPrefillArgs p) {
 // causal GQA attention over the prompt (reference.py:645-677)
 // ---------------------------------------------------------------------------------------
 //
-// scores = bf16(bf16(q . k) * scale), masked above the diagonal; p = bf16(softmax_fp32);
-// o = bf16(p @ V); out = bf16(o * bf16(gate_fn(gate))). The bf16 rounding of p needs the
-// row's final max and sum, so the keys are visited twice: pass 1 finds (max, sum), pass 2
-// forms p and accumulates p V. A workgroup owns 16 query positions of one KV head; wave w is
-// query head 4 g + w. Products run on v_mfma_f32_16x16x32_bf16 (query rows x keys, then
-// query rows x head dims); keys are staged 64 at a time, V transposed for its B operand.
+// scores = bf16(bf16(q . k) * scale), masked above the diagonal; p = softmax over fp32; o = p V
+// with p rounded to bf16 for the product; out = bf16(bf16(o) * bf16(gate_fn(gate))).
+//
+// A workgroup owns 32 query positions of one KV head. Wave w is query head 4 g + w % 4 and key
+// set w / 4, which takes every other 32 keys; the two sets' (m, l, O) are merged at the end.
+// Keys and values pass through LDS in blocks of 64 (32 for each set), two buffers, filled by
+// global_load_lds a block ahead. One pass over the keys, on v_mfma_f32_32x32x16_bf16 with the
+// keys as rows: S^T = K Q^T leaves a query's scores in its lane's registers (column
+// lane % 32), so max and sum need one exchange with lane + 32, and exp(S^T) is at once the B
+// operand of O^T = V^T P^T: lane half h holds keys 4 h + {0..3, 8..11} of 16, and V^T comes in
+// that key order from ds_read_tr16_b64, which transposes 4 keys x 16 dims of the row-major
+// tile. K's 16-byte chunks are XORed with key % 16 and V's with 4 (key % 8), so that both
+// reads spread over the banks.
+//
+// p is exp(s - m) with m a running maximum that moves only when a block exceeds it by more
+// than 2^8 (p and l then stay far inside fp32); bf16(p) has the relative rounding that the
+// normalised bf16 probability has, and l sums the unrounded p. The first 32 positions, whose
+// few weights are large, know their sum before the product and round p / l as the reference
+// does. A row's result depends only on its own scores in blocks of 32 keys from key 0, so a
+// prompt filled in chunks equals one pass.
+//
+// The next block's K products run between this block's softmax, so the VALU is hidden (without
+// it the kernel takes as long). What bounds it is LDS: per 64 keys a CU reads 256 KB of operands and
+// writes 64 KB, for 2048 cycles of products in about 4900 (without the DMA 20 % faster, without
+// either product 22 %). Causal prompts, us before (two passes over the keys, 16 query rows to a
+// wave) -> now: 8192 tokens 3106 -> 573 (959 TFLOP/s), 717 tokens 114 -> 38; 2000 tokens after
+// 20 000 keys 675 (1019 TFLOP/s). Measured and not kept: 64 positions to a workgroup and no key
+// sets (8192 tokens 562, 717 tokens 55), two barriers with K and V two blocks ahead (595),
+// reading an operand right before its product (597).
 
 constexpr int kAtKeys = 64;
-constexpr int kKsPitch = kHd + 8;
-constexpr int kVtPitch = kAtKeys + 8;
-constexpr int kPtPitch = kAtKeys + 8;
+constexpr int kAtTile = kAtKeys * kHd * 2;  // bytes of a K or V block
+constexpr int kAtThreads = 512;
+constexpr int kAtMl = 4 * kAtTile;          // byte offset of the sets' (m, l) exchange
+constexpr int kAtLds = kAtMl + 8 * 32 * 8;
+constexpr float kLog2e = 1.44269504088896f;
+constexpr int kAtPow2Scale = 1;  // scale is a positive power of two: bf16(s * scale) is exact
+constexpr int kAtVecGate = 2;    // gate rows allow 8-byte loads
+constexpr int kAtVecOut = 4;     // out rows allow 8-byte stores
 
-__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(DfAttnPrefillArgs p) {
-  __shared__ __align__(16) uint16_t Ks[kAtKeys * kKsPitch];
-  __shared__ __align__(16) uint16_t Vt[kHd * kVtPitch];
-  __shared__ __align__(16) uint16_t Pt[4][16 * kPtPitch];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = blockIdx.y, h = g * 4 + wave;
-  const int t0 = blockIdx.x * 16;
-  const int rq = lane & 15, kq = lane >> 4;
-  // A operands of q . k: row rq, dims 32 ds + 8 kq .. + 8
-  uint4 qa[8];
-  {
-    const int t = t0 + rq;
-#pragma unroll
-    for (int ds = 0; ds < 8; ++ds)
-      qa[ds] = t < p.tokens
-                   ? *reinterpret_cast<const uint4*>(p.q + ((size_t)t * p.num_q_heads + h) * kHd + ds * 32 + kq * 8)
-                   : make_uint4(0u, 0u, 0u, 0u);
-  }
-  const int last_t = min(t0 + 16, p.tokens) - 1;
-  const int nkeys = p.pos0 + last_t + 1;  // keys any row of the block attends
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+DF_DEVICE s16x4 read_tr(uint32_t at) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(at));
+}
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+
+__global__ __launch_bounds__(kAtThreads, 1) void attn_prefill_kernel(DfAttnPrefillArgs p, int flags) {
+  extern __shared__ __align__(1024) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, q = lane & 31;
+  // KV head fastest, so that an XCD (workgroups i mod 8) reads one head's keys; the last
+  // positions, which have the most keys, first
+  const int g = blockIdx.x % p.num_kv_heads;
+  const int qblocks = (p.tokens + 31) / 32;
+  const int h = g * 4 + (wave & 3), kset = wave >> 2, t0 = (qblocks - 1 - blockIdx.x / p.num_kv_heads) * 32;
+  const uint32_t lds0 = lds_offset(smem);
+
+  const int nkeys = p.pos0 + min(t0 + 32, p.tokens);  // keys any row of the block attends
   const int nkb = (nkeys + kAtKeys - 1) / kAtKeys;
-  const uint16_t* kbase = p.k_cache + (size_t)g * p.max_len * kHd;
-  const uint16_t* vbase = p.v_cache + (size_t)g * p.max_len * kHd;
-  // this lane's rows of the 16 x 16 products: 4 kq + r, at positions pos0 + t0 + 4 kq + r
-  float m[4], l[4];
+  const unsigned char* kbase = reinterpret_cast<const unsigned char*>(p.k_cache + (size_t)g * p.max_len * kHd);
+  const unsigned char* vbase = reinterpret_cast<const unsigned char*>(p.v_cache + (size_t)g * p.max_len * kHd);
+  constexpr int kOps = kAtTile / (kAtThreads * 16);  // DMAs per wave and block of K or V
+  constexpr int kAhead = 2;                          // LDS operands in flight
+  // This thread's chunk of DMA i: key 16 i + tid / 32 of the block, slot tid % 32. Full blocks go
+  // by a uniform base and a per-thread offset; in the last one keys past the end repeat the last.
+  const uint32_t krow = (tid >> 5) * (kHd * 2), kchunk = ((tid & 31) ^ (tid >> 5)) << 4;
+  const uint32_t vchunk = ((tid & 31) ^ (((tid >> 5) & 7) << 2)) << 4;
+  auto issue = [&](const unsigned char* base, uint32_t chunk, int kb, uint32_t at) {
+    const unsigned char* block = base + (size_t)kb * kAtTile;
+    if (kb * kAtKeys + kAtKeys <= nkeys) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    m[r] = -INFINITY;
-    l[r] = 0.0f;
+      for (int i = 0; i < kOps; ++i)
+        dma16s(block + i * (16 * kHd * 2), krow + chunk, at + i * (kAtThreads * 16));
+    } else {
+#pragma unroll
+      for (int i = 0; i < kOps; ++i) {
+        const int key = min(i * 16 + (tid >> 5), nkeys - 1 - kb * kAtKeys);
+        dma16s(block, key * (kHd * 2) + chunk, at + i * (kAtThreads * 16));
+      }
+    }
+  };
+  auto issue_k = [&](int kb) { issue(kbase, kchunk, kb, lds0 + (kb & 1) * 2 * kAtTile + wave * 1024); };
+  auto issue_v = [&](int kb) { issue(vbase, vchunk, kb, lds0 + (kb & 1) * 2 * kAtTile + kAtTile + wave * 1024); };
+  // B operands of K Q^T: step n takes dims 16 n + 8 half ..+7. Rows past the prompt repeat its last
+  // one and are not stored.
+  uint4 qf[16];
+  {
+    const uint16_t* src = p.q + ((size_t)min(t0 + q, p.tokens - 1) * p.num_q_heads + h) * kHd + half * 8;
+#pragma unroll
+    for (int n = 0; n < 16; ++n) qf[n] = *reinterpret_cast<const uint4*>(src + n * 16);
+#pragma unroll
+    for (int n = 0; n < 16; ++n)
+      asm volatile("" : "+v"(qf[n].x), "+v"(qf[n].y), "+v"(qf[n].z), "+v"(qf[n].w));  // waited for here
   }
+  issue_k(0);
+  issue_v(0);
+  if (nkb > 1) issue_k(1);
+  const int pos = p.pos0 + t0 + q;
+  const int pos_lo = p.pos0 + t0, pos_hi = pos_lo + 31;  // the wave's positions
+  const bool pow2 = flags & kAtPow2Scale;
+  const float cexp = pow2 ? p.scale * kLog2e : kLog2e;
 
-  // Key block kb's K (and V) rows: loaded into registers one block ahead, stored into LDS
-  // once the previous block's products are done with it. V is stored transposed (Vt[d][key],
-  // the B operand of p V): thread (dim pair dp = tid % 128, half kh = tid / 128) loads dims
-  // 2 dp, 2 dp + 1 of keys 32 kh + 8 q + j (4-byte loads, coalesced across the lanes) and
-  // writes each dim's 8 keys with one 16-byte store.
-  uint4 kr[8];
-  uint32_t vr[32];
-  auto load_rows = [&](uint4 (&rr)[8], const uint16_t* src, int kb) {  // K rows
+  f32x16 o[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {  // 64 keys x 32 chunks of 16 bytes
-      const int ch = tid + 256 * i, key = ch >> 5, cc = ch & 31;
-      const int kg = kb * kAtKeys + key;
-      rr[i] = make_uint4(0u, 0u, 0u, 0u);
-      if (kg < nkeys) rr[i] = *reinterpret_cast<const uint4*>(src + (size_t)kg * kHd + cc * 8);
-    }
-  };
-  auto put_k = [&]() {
+  for (int db = 0; db < 8; ++db)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int ch = tid + 256 * i, key = ch >> 5, cc = ch & 31;
-      *reinterpret_cast<uint4*>(&Ks[key * kKsPitch + cc * 8]) = kr[i];
-    }
-  };
-  const int vdp = tid & 127, vkh = tid >> 7;
-  auto load_v = [&](int kb) {
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
-      const int kg = kb * kAtKeys + 32 * vkh + i;
-      vr[i] = kg < nkeys ? *reinterpret_cast<const uint32_t*>(vbase + (size_t)kg * kHd + 2 * vdp) : 0u;
-    }
-  };
-  auto put_v = [&]() {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint32_t* w = vr + 8 * q;
-      const uint4 lo = make_uint4((w[0] & 0xFFFFu) | (w[1] << 16), (w[2] & 0xFFFFu) | (w[3] << 16),
-                                  (w[4] & 0xFFFFu) | (w[5] << 16), (w[6] & 0xFFFFu) | (w[7] << 16));
-      const uint4 hi = make_uint4((w[0] >> 16) | (w[1] & 0xFFFF0000u), (w[2] >> 16) | (w[3] & 0xFFFF0000u),
-                                  (w[4] >> 16) | (w[5] & 0xFFFF0000u), (w[6] >> 16) | (w[7] & 0xFFFF0000u));
-      const int key0 = 32 * vkh + 8 * q;
-      *reinterpret_cast<uint4*>(&Vt[(2 * vdp) * kVtPitch + key0]) = lo;
-      *reinterpret_cast<uint4*>(&Vt[(2 * vdp + 1) * kVtPitch + key0]) = hi;
-    }
-  };
-  // scores of key block kb for this lane: s[sb][r] (key kb*64 + 16 sb + lane % 16)
-  auto scores = [&](int kb, float (&s)[4][4]) {
-#pragma unroll
-    for (int sb = 0; sb < 4; ++sb) {
-      df_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ds = 0; ds < 8; ++ds) {
-        const uint4 b = *reinterpret_cast<const uint4*>(&Ks[(sb * 16 + rq) * kKsPitch + ds * 32 + kq * 8]);
-        acc = mfma(qa[ds], b, acc);
-      }
-      const int key = kb * kAtKeys + sb * 16 + rq;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int pos = p.pos0 + t0 + kq * 4 + r;
-        s[sb][r] = key <= pos ? round_bf(round_bf(acc[r]) * p.scale) : -INFINITY;
-      }
-    }
-  };
+    for (int e = 0; e < 16; ++e) o[db][e] = 0.f;
+  float m = -INFINITY, l = 0.0f;  // m: the maximum in use, in units of log2(e) (scaled)
 
-  // ---- pass 1: row max and sum --------------------------------------------------------
-  load_rows(kr, kbase, 0);
+  // LDS addresses of this lane: K row q, chunk half ^ (q % 16) (step n: ^ 32 n); V key
+  // 4 half + (lane % 16) / 4, dims 16 ((lane / 16) % 2) + 4 (lane % 4) (dim block db: ^ 64 db)
+  const uint32_t ka = q * (kHd * 2) + ((half ^ (q & 15)) << 4);
+  const int vkey = 4 * half + ((lane & 15) >> 2);
+  const uint32_t va = vkey * (kHd * 2) + (vkey << 6) + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+
+  // blocks in which this set has keys that some row attends
+  const int live = pos_hi < kset * 32 ? 0 : min(nkb, (pos_hi - kset * 32) / kAtKeys + 1);
+  auto k_at = [&](int kb) {
+    uint32_t at = lds0 + (kb & 1) * 2 * kAtTile + kset * (32 * kHd * 2) + ka;
+    asm volatile("" : "+v"(at));  // the 16 addresses are made from it block by block: kept, they would spill
+    return at;
+  };
+  auto read_k = [&](uint32_t at, int n) { return *reinterpret_cast<const lds_u32x4*>(at ^ (n << 5)); };
+  // lane: query q, keys key0 + (e % 4) + 8 (e / 4) + 4 half
+  auto mask = [&](f32x16& s, int kb) {
+    const int key0 = kb * kAtKeys + kset * 32;
+    if (key0 + 31 > pos_lo) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        s[e] = key0 + (e & 3) + 8 * (e >> 2) + 4 * half <= pos ? s[e] : -INFINITY;
+    }
+  };
+  auto prob = [&](float r, float mc) { return __builtin_amdgcn_exp2f(fmaf(r, cexp, -mc)); };
+  // One block: the products of the next block's scores (sn) run between the VALU work of this
+  // block's softmax (s), two scores a product; then this block's values.
+  // After the last block the products read a stale buffer and their result is dropped.
+  auto step = [&](f32x16& s, int kb) {
+    u32x4 kf[kAhead];
+    f32x16 sn;
+    const uint32_t kat = k_at(kb + 1);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sn[e] = 0.f;
+#pragma unroll
+    for (int n = 0; n < kAhead; ++n) kf[n] = read_k(kat, n);
+    __builtin_amdgcn_sched_barrier(0);
+    auto product = [&](int n) {
+      sn = mfma32(__builtin_bit_cast(uint4, kf[n % kAhead]), qf[n], sn);
+      if (n + kAhead < 16) kf[n % kAhead] = read_k(kat, n + kAhead);
+    };
+    float mx = -INFINITY;
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      product(n);
+      const uint32_t two = pack_bf16(s[2 * n], s[2 * n + 1]);
+      s[2 * n] = __uint_as_float(two << 16);
+      s[2 * n + 1] = __uint_as_float(two & 0xFFFF0000u);
+      if (!pow2) {
+        s[2 * n] = round_bf(s[2 * n] * p.scale);
+        s[2 * n + 1] = round_bf(s[2 * n + 1] * p.scale);
+      }
+      mx = fmaxf(fmaxf(mx, s[2 * n]), s[2 * n + 1]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * cexp;
+    const bool move = mx > m + 8.0f;
+    if (__any(move)) {
+      const float mn = move ? mx : m;
+      const float alpha = move ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < 8; ++db)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[db][e] *= alpha;
+    }
+    const float mc = m == -INFINITY ? 0.0f : m;
+    float sum = 0.0f;
+    uint32_t pk[8];
+#pragma unroll
+    for (int n = 8; n < 16; ++n) {
+      product(n);
+      const int e = 2 * (n - 8);
+      const float p0 = prob(s[e], mc), p1 = prob(s[e + 1], mc);
+      sum += p0 + p1;
+      pk[n - 8] = pack_bf16(p0, p1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (kb == 0 && kset == 0 && pos_lo < 32) {
+      // a row whose keys all lie in the first 32 is normalised before the rounding
+      const float total = sum + __shfl_xor(sum, 32, 64);
+      const float norm = pos >= 32 ? 1.0f : total == 0.0f ? 0.0f : 1.0f / total;
+      if (pos < 32) sum = 0.5f;
+#pragma unroll
+      for (int e = 0; e < 16; e += 2) pk[e / 2] = pack_bf16(prob(s[e], mc) * norm, prob(s[e + 1], mc) * norm);
+    }
+    l += sum;
+    mask(sn, kb + 1);
+    // O^T += V^T P^T: keys 16 kk + 4 half + {0..3, 8..11} are the lane's values 8 kk .. 8 kk + 7
+    uint32_t vat = lds0 + (kb & 1) * 2 * kAtTile + kAtTile + kset * (32 * kHd * 2) + va;
+    asm volatile("" : "+v"(vat));
+    auto read_v = [&](int u) {  // unit u: dims 32 (u / 2) .. + 31, keys 16 (u % 2) .. + 15
+      const uint32_t at = (vat ^ ((u >> 1) << 6)) + (u & 1) * (16 * kHd * 2);
+      const uint2 a0 = __builtin_bit_cast(uint2, read_tr(at));
+      const uint2 a1 = __builtin_bit_cast(uint2, read_tr(at + 8 * (kHd * 2)));
+      return make_uint4(a0.x, a0.y, a1.x, a1.y);
+    };
+    uint4 vf[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) vf[u] = read_v(u);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int kk = u & 1;
+      const uint4 pv = make_uint4(pk[4 * kk], pk[4 * kk + 1], pk[4 * kk + 2], pk[4 * kk + 3]);
+      o[u >> 1] = mfma32(vf[u % kAhead], pv, o[u >> 1]);
+      if (u + kAhead < 16) vf[u % kAhead] = read_v(u + kAhead);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    s = sn;
+  };
+  f32x16 sa;
+  wait_vm<0>();
+  __syncthreads();
+  if (live > 0) {
+    const uint32_t kat = k_at(0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sa[e] = 0.f;
+#pragma unroll
+    for (int n = 0; n < 16; ++n) sa = mfma32(__builtin_bit_cast(uint4, read_k(kat, n)), qf[n], sa);
+    mask(sa, 0);
+  }
   for (int kb = 0; kb < nkb; ++kb) {
-    put_k();
-    __syncthreads();
-    if (kb + 1 < nkb) load_rows(kr, kbase, kb + 1);
-    float s[4][4];
-    scores(kb, s);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float mx = fmaxf(fmaxf(s[0][r], s[1][r]), fmaxf(s[2][r], s[3][r]));
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-      const float mn = fmaxf(m[r], mx);
-      float sum = 0.0f;
-#pragma unroll
-      for (int sb = 0; sb < 4; ++sb) sum += s[sb][r] == -INFINITY ? 0.0f : expf(s[sb][r] - mn);
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) sum += __shfl_xor(sum, off, 64);
-      l[r] = (m[r] == -INFINITY ? 0.0f : l[r] * expf(m[r] - mn)) + sum;
-      m[r] = mn;
-    }
-    __syncthreads();
+    wait_vm<0>();     // this wave's part of K (kb + 1) and V (kb) is in LDS
+    __syncthreads();  // every wave's is, and every wave is done with K (kb) and V (kb - 1)
+    if (kb + 2 < nkb) issue_k(kb + 2);
+    if (kb + 1 < nkb) issue_v(kb + 1);
+    if (kb < live) step(sa, kb);
   }
+  l += __shfl_xor(l, 32, 64);  // the two halves summed their own keys
 
-  // ---- pass 2: p = bf16(exp(s - max) / sum), o += p V ----------------------------------
-  df_f32x4 o[16];
+  // ---- the sets' merge: each set finishes half of the head's dims -----------------------
+  // The gates this wave will need (rows 2 i + lane / 32, 4 dims) are loaded ahead.
+  const int d0 = kset * 128 + (lane & 31) * 4;
+  uint2 gr[16];
 #pragma unroll
-  for (int db = 0; db < 16; ++db) o[db] = df_f32x4{0.f, 0.f, 0.f, 0.f};
-  uint16_t* pt = Pt[wave];
-  load_rows(kr, kbase, 0);
-  load_v(0);
-  for (int kb = 0; kb < nkb; ++kb) {
-    put_k();
-    put_v();
-    __syncthreads();
-    if (kb + 1 < nkb) {
-      load_rows(kr, kbase, kb + 1);
-      load_v(kb + 1);
+  for (int i = 0; i < 16; ++i) {
+    const int t = min(t0 + 2 * i + half, p.tokens - 1);
+    const uint16_t* src = p.gate + (size_t)t * p.ld_gate + h * p.gate_head_stride + d0;
+    if (flags & kAtVecGate) {
+      gr[i] = *reinterpret_cast<const uint2*>(src);
+    } else {
+      gr[i].x = src[0] | (static_cast<uint32_t>(src[1]) << 16);
+      gr[i].y = src[2] | (static_cast<uint32_t>(src[3]) << 16);
     }
-    float s[4][4];
-    scores(kb, s);
-#pragma unroll
-    for (int sb = 0; sb < 4; ++sb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float pr = s[sb][r] == -INFINITY ? 0.0f : expf(s[sb][r] - m[r]) / l[r];
-        pt[(kq * 4 + r) * kPtPitch + sb * 16 + rq] = f2bf(pr);
-      }
-    __syncthreads();  // p rows are read back by other lanes of the wave in the A layout
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const uint4 pa = *reinterpret_cast<const uint4*>(&pt[rq * kPtPitch + ks * 32 + kq * 8]);
-#pragma unroll
-      for (int db = 0; db < 16; ++db) {
-        const uint4 b = *reinterpret_cast<const uint4*>(&Vt[(db * 16 + rq) * kVtPitch + ks * 32 + kq * 8]);
-        o[db] = mfma(pa, b, o[db]);
-      }
-    }
-    __syncthreads();
   }
-
-  // ---- epilogue: bf16(o) * bf16(gate_fn(gate)) ----------------------------------------
+  __syncthreads();  // every wave is done with the keys and values
+  float2* ml = reinterpret_cast<float2*>(smem + kAtMl);
+  if (half == 0) ml[wave * 32 + q] = make_float2(m, l);
+  const int partner = wave ^ 4;
+  float4* give = reinterpret_cast<float4*>(smem + partner * 16384) + lane;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int t = t0 + kq * 4 + r;
-    if (t >= p.tokens) continue;
-    const uint16_t* gr = p.gate + (size_t)t * p.ld_gate + h * p.gate_head_stride;
-    uint16_t* orow = p.out + (size_t)t * p.ld_out + h * kHd;
+  for (int db = 0; db < 4; ++db)
 #pragma unroll
-    for (int db = 0; db < 16; ++db) {
-      const int d = db * 16 + rq;
-      const float gx = bf2f(gr[d]);
-      const float gv = round_bf(p.gate_kind == 0 ? sigmoid(gx) : silu(gx));
-      orow[d] = f2bf(round_bf(o[db][r]) * gv);
+    for (int e = 0; e < 4; ++e) {
+      const f32x16 v = kset ? o[db] : o[4 + db];
+      give[(db * 4 + e) * 64] = make_float4(v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]);
+    }
+  __syncthreads();
+  const float2 other = ml[partner * 32 + q];
+  const float mm = fmaxf(m, other.x);
+  const float a_own = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mm);
+  const float a_oth = other.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(other.x - mm);
+  // set 0's term first, whichever set adds them
+  const float l0 = kset ? a_oth * other.y : a_own * l, l1 = kset ? a_own * l : a_oth * other.y;
+  const float den = l0 + l1, inv = den == 0.0f ? 0.0f : 1.0f / den;
+  const float w_own = a_own * inv, w_oth = a_oth * inv;
+  const float4* take = reinterpret_cast<const float4*>(smem + wave * 16384) + lane;
+  float y[4][16];
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const f32x16 v = kset ? o[4 + db] : o[db];
+      const float4 u = take[(db * 4 + e) * 64];
+      const float uu[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[db][4 * e + i] = fmaf(v[4 * e + i], w_own, uu[i] * w_oth);
+    }
+  // bf16(o) through this wave's part of LDS to whole rows, times bf16(gate_fn(gate))
+  constexpr int kPitch = 128 * 2 + 16;
+  unsigned char* ot = smem + wave * 16384;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      *reinterpret_cast<uint2*>(ot + q * kPitch + (db * 32 + e * 8 + half * 4) * 2) =
+          make_uint2(pack_bf16(y[db][4 * e], y[db][4 * e + 1]), pack_bf16(y[db][4 * e + 2], y[db][4 * e + 3]));
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int t = t0 + 2 * i + half;
+    if (t >= p.tokens) break;
+    float v[4], gx[4];
+    load4(reinterpret_cast<const uint16_t*>(ot + (2 * i + half) * kPitch) + (lane & 31) * 4, v);
+    load4(reinterpret_cast<const uint16_t*>(&gr[i]), gx);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] *= round_bf(p.gate_kind == 0 ? sigmoid(gx[j]) : silu(gx[j]));
+    uint16_t* orow = p.out + (size_t)t * p.ld_out + h * kHd + d0;
+    if (flags & kAtVecOut) {
+      store4(orow, v);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) orow[j] = f2bf(v[j]);
     }
   }
 }
@@ -1215,8 +1355,16 @@ int df_attention_prefill(const DfAttnPrefillArgs* a, hipStream_t stream) {
   if (!aligned16(a->q) || !aligned16(a->k_cache) || !aligned16(a->v_cache) || a->ld_out < a->num_q_heads * kHd ||
       a->gate_kind < 0 || a->gate_kind > 1)
     return DF_BAD_ARGUMENT;
-  const int qb = (a->tokens + 15) / 16;
-  hipLaunchKernelGGL(attn_prefill_kernel, dim3(qb, a->num_kv_heads), dim3(256), 0, stream, *a);
+  int e = 0;
+  const bool pow2 = a->scale > 0.0f && frexpf(a->scale, &e) == 0.5f;
+  auto mult = [](const void* ptr, int ld, int align) {
+    return (reinterpret_cast<uintptr_t>(ptr) % align) == 0 && ld % (align / 2) == 0;
+  };
+  const int flags = (pow2 ? kAtPow2Scale : 0) |
+                    (mult(a->gate, a->ld_gate, 8) && a->gate_head_stride % 4 == 0 ? kAtVecGate : 0) |
+                    (mult(a->out, a->ld_out, 8) ? kAtVecOut : 0);
+  hipLaunchKernelGGL(attn_prefill_kernel, dim3((a->tokens + 31) / 32 * a->num_kv_heads), dim3(kAtThreads), kAtLds,
+                     stream, *a, flags);
   DF_RETURN_LAUNCH_STATUS();
 }
 

@@ -193,6 +193,50 @@ def test_gated_rms_norm_rows():
     close(got, want, what="gated norm rows")
 
 
+def _attention_expression(q, k, v, gate, pos0, scale, swish):
+    """The reference's rounding in fp32: bf16 scores, bf16 softmax, bf16 output, bf16 gate."""
+    p, hq, _ = q.shape
+    out = torch.empty((p, hq, 256))
+    keep = torch.arange(pos0 + p)[None] <= pos0 + torch.arange(p)[:, None]
+    for h in range(hq):
+        kk, vv = k[h // 4, :pos0 + p].float(), v[h // 4, :pos0 + p].float()
+        s = ((q[:, h].float() @ kk.t()).to(torch.bfloat16).float() * scale).to(torch.bfloat16).float()
+        w = torch.softmax(s.masked_fill(~keep, float("-inf")), -1).to(torch.bfloat16).float()
+        out[:, h] = (w @ vv).to(torch.bfloat16).float()
+    g = gate.float()
+    g = (g * torch.sigmoid(g) if swish else torch.sigmoid(g)).to(torch.bfloat16).float()
+    return (out * g).to(torch.bfloat16).reshape(p, -1)
+
+
+# row blocks of 32 positions, key blocks of 64 in two sets of 32, the first 32 positions, later
+# chunks; a scale that is no power of two; gate and output rows that allow no 8-byte access
+@pytest.mark.parametrize("tokens,pos0,scale,swish,shift", [
+    (1, 0, 1 / 16, False, 0), (31, 0, 1 / 16, True, 0), (33, 0, 0.07, False, 0), (64, 0, 1 / 16, False, 1),
+    (97, 0, 0.05, True, 3), (1, 31, 1 / 16, False, 0), (2, 31, 1 / 16, False, 0), (40, 30, 1 / 16, False, 0),
+    (1, 64, 1 / 16, False, 0), (70, 200, 1 / 16, False, 2), (130, 63, 0.3, False, 0)])
+def test_attention_prefill_edges(tokens, pos0, scale, swish, shift):
+    print(f"attention prefill {tokens} at {pos0}", flush=True)
+    from deltaforge_amd import prefill as P
+
+    gen = torch.Generator().manual_seed(1000 * tokens + pos0)
+    max_len = pos0 + tokens + 5
+    q = torch.randn((tokens, 8, 256), generator=gen).to(torch.bfloat16)
+    k, v = (torch.randn((2, max_len, 256), generator=gen).to(torch.bfloat16) for _ in range(2))
+    k[:, pos0 + tokens:], v[:, pos0 + tokens:] = float("nan"), float("nan")  # rows past the prompt are not read
+    wide = torch.randn((tokens, shift + 8 * 512), generator=gen).to(torch.bfloat16)
+    gate = wide[:, shift:]
+    kd, vd, qd, gd = k.to(DEV), v.to(DEV), q.to(DEV), wide.to(DEV)[:, shift:]
+    out = torch.zeros((tokens, 8 * 256 + 2 * shift), dtype=torch.bfloat16, device=DEV)[:, shift:shift + 8 * 256]
+    got = P.attention_prefill(qd, kd, vd, gd, gate_head_stride=512, pos0=pos0, gate_kind=int(swish), scale=scale, out=out)
+    heads = torch.stack([gate[:, h * 512:h * 512 + 256] for h in range(8)], 1)
+    close(got, _attention_expression(q, k, v, heads, pos0, scale, swish), what="attention", flip_frac=5e-3)
+    if tokens > 1:  # later rows as a chunk of their own
+        at = tokens // 3
+        part = P.attention_prefill(qd[at:].contiguous(), kd, vd, gd[at:], gate_head_stride=512, pos0=pos0 + at,
+                                   gate_kind=int(swish), scale=scale)
+        assert torch.equal(part, got[at:])
+
+
 # -- layers and the model -------------------------------------------------------------------
 
 
