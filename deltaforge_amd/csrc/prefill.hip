@@ -129,6 +129,14 @@ DF_DEVICE uint32_t lds_offset(const void* p) {
   return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const lds_byte*)p));
 }
 
+// A transposing LDS read: each 16 lanes give the addresses of four rows of 16 values, 4 lanes a
+// row (8 bytes each), and lane i gets column i of the four.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+DF_DEVICE s16x4 read_tr(uint32_t at) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(at));
+}
+
 template <int EPI, int RB, int CP, int WN, int NBUF, bool WREG>
 __global__ __launch_bounds__(128 * WN, 1) void int4_gemm_kernel(DfInt4GemmArgs p, GemmGeom geo) {
   using SH = GemmShape<RB, CP, WN, NBUF, WREG>;
@@ -427,356 +435,456 @@ __global__ __launch_bounds__(256) void conv_ring_update_kernel(const uint16_t* _
 //   S <- exp(g_t) S;  delta_t = beta_t (v_t - S^T k_t);  S <- S + k_t delta_t^T;  o_t = S^T q_t
 // is, exactly in real arithmetic:
 //   A'[t][j] = beta_t exp(gamma_t - gamma_j) (k_t . k_j), j < t      (strictly lower)
-//   [Wv | Wk] = (I + A')^-1 [diag(beta) V | diag(beta e^gamma) K]      (forward substitution)
-//   delta    = Wv - Wk S0
+//   T        = (I + A')^-1                                            (unit lower)
 //   QK[t][j] = exp(gamma_t - gamma_j) (q_t . k_j), j <= t
-//   O        = O_loc + Qx S0,   O_loc = QK Wv,   Qx = diag(e^gamma) Q - QK Wk
-//   S_C      = e^gamma_C S0 + Kd^T delta,   Kd = diag(exp(gamma_C - gamma)) K
-// with q, k the L2-normalised rows (q also / sqrt(Dk)). Everything but the three products
-// with S0 is independent of the state, so it runs for every (chunk, head) at once
-// (delta_prep_kernel, 2048 workgroups at 4096 tokens). The scan kernel then walks the chunks
-// in order with the state slice in LDS and does only O, delta and the state update.
-// Padding tokens past the prompt get g = beta = 0 and q = k = v = 0, which changes nothing.
+//   delta    = T R,  R = diag(beta) V - diag(beta e^gamma) K S0
+//   O        = diag(e^gamma) Q S0 + QK delta
+//   S_C      = e^gamma_C S0 + K^T diag(exp(gamma_C - gamma)) delta
+// with q, k the L2-normalised rows (q also / sqrt(Dk)). T and QK do not depend on the state:
+// delta_prep_kernel forms them for every (chunk, value head) at once, with the per-token
+// factors. delta_scan_kernel then walks the chunks in order.
+//
+// The rows are kept raw, as the bf16 the conv wrote, and their norms go into the per-token
+// factors. So K K^T and Q K^T are exact products of bf16 on the matrix core with fp32 sums, and
+// K S0, Q S0 and K^T delta are too once the fp32 operand is written as three bf16 (8 + 8 + 8
+// significant bits, every remainder exact): three products at 1 / 16 of the fp32 product's
+// cost. T R and QK delta, where both sides are fp32, stay on v_mfma_f32_16x16x4_f32.
+// Padding tokens past the prompt get g = beta = 0 (their rows repeat the last token's), so their
+// rows of A', R and delta are zero and the state does not see them.
 
-constexpr int kCk = 64;          // tokens per chunk
-constexpr int kDk = 128;         // key (and value) head dim
-constexpr int kPitch = kDk + 4;  // fp32 row pitch in LDS
-constexpr int kMat = kCk * kDk;  // floats of one chunk matrix in the scratch
-constexpr int kPrepMats = 5;     // O_loc, Qx, Wv, Wk, Kd
+constexpr int kCk = 64;             // tokens per chunk
+constexpr int kDk = 128;            // key (and value) head dim
+constexpr int kBlk = 256;           // floats of a 16 x 16 block
+constexpr int kTri = 10;            // lower block triangle of 4 x 4 blocks
+// One (chunk, value head) in the scratch, in floats: T's blocks (b, c <= b) at b (b + 1) / 2 + c,
+// each [j / 4][t][j % 4] (the fp32 product's A operand, lane by lane), QK's likewise, then
+// per token beta e^gamma rk | beta | exp(gamma_C - gamma) rk | e^gamma rq / sqrt(Dk), then e^gamma_C.
+constexpr int kPrepQk = kTri * kBlk;
+constexpr int kPrepTok = 2 * kTri * kBlk;
+constexpr int kPrepEc = kPrepTok + 4 * kCk;
+constexpr int kPrepFloats = kPrepEc + 16;  // (16 copies: a vector load, in order with the others)
 
-DF_DEVICE size_t prep_base(int chunk, int h, int hv) { return ((size_t)chunk * hv + h) * kPrepMats * kMat; }
+DF_DEVICE size_t prep_base(int chunk, int h, int hv) { return ((size_t)chunk * hv + h) * kPrepFloats; }
+DF_DEVICE int tri(int b, int c) { return b * (b + 1) / 2 + c; }
+DF_DEVICE df_f32x4 mfma4(float a, float b, df_f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+// acc += A B over one 16-wide block of the sum: a = A[row][4 q ..+3], b = B[4 q ..+3][col]
+DF_DEVICE df_f32x4 mfma16(const float4& a, const float4& b, df_f32x4 acc) {
+  acc = mfma4(a.x, b.x, acc);
+  acc = mfma4(a.y, b.y, acc);
+  acc = mfma4(a.z, b.z, acc);
+  return mfma4(a.w, b.w, acc);
+}
+DF_DEVICE float4 as_f4(const uint4& v) { return __builtin_bit_cast(float4, v); }
+// 16 bytes from an address that may be only 4-byte aligned.
+DF_DEVICE uint4 load16u(const uint16_t* p, bool aligned) {
+  if (aligned) return *reinterpret_cast<const uint4*>(p);
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(p);
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
 
+// Four waves; wave w owns tokens 16 w .. + 15. K K^T and Q K^T on 16 x 16 x 32 products (their
+// diagonals and Q Q^T's give the norms), A' into LDS, then T block by block: each wave inverts
+// its diagonal block by forward substitution (lane = column), and the blocks below follow by
+// diagonals, T_ba = -T_bb sum_{a <= c < b} A'_bc T_ca. 4096 tokens: 507 us with fp32 VALU products
+// of all of R's columns and 335 MB of results -> 45 us and 44 MB.
 struct PrepLds {
-  float Q[kCk][kPitch];
-  float K[kCk][kPitch];
-  float V[kCk][kPitch];
-  float At[kCk][kCk];   // A' transposed: At[j][t] = A'[t][j] (beta_t-scaled, decayed, strictly lower)
-  float QK[kCk][kCk];   // decayed, lower with the diagonal
-  float gam[kCk], beta[kCk], eg[kCk], dec[kCk];
+  uint4 k[kCk * 16], q[kCk * 16];   // raw rows, 16-byte chunk c of row t in slot c ^ (t % 16)
+  float a[kTri][16][20];            // A' blocks, [t][j]
+  float tt[kTri][16][20];           // T blocks transposed, [j][t]
+  float td[4][16][20];              // T's diagonal blocks, [t][j]
+  float pt[3][16][20];              // a product on its way from result to operand, transposed
+  float gam[kCk], beta[kCk], nk[kCk], nq[kCk];
 };
 
-__global__ __launch_bounds__(256) void delta_prep_kernel(DfDeltaPrefillArgs p, float* __restrict__ scratch) {
+__global__ __launch_bounds__(256) void delta_prep_kernel(DfDeltaPrefillArgs p, float* __restrict__ scratch, int aligned) {
   __shared__ __align__(16) PrepLds L;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int chunk = blockIdx.x, h = blockIdx.y;
   const int c0 = chunk * kCk;
   const int kh = h / (p.num_v_heads / p.num_k_heads);
   const int key_dim = p.num_k_heads * kDk;
-  const int qoff = kh * kDk, koff = key_dim + kh * kDk, voff = 2 * key_dim + h * kDk;
-  const float qscale = sqrtf(static_cast<float>(kDk));
+  const int n16 = lane & 15, q4 = lane >> 4;
+  float* base = scratch + prep_base(chunk, h, p.num_v_heads);
 
-  // ---- normalised q, k rows; v rows; gates --------------------------------------------
-  // wave w: tokens 16 w ..; all 16 tokens' loads are issued before any is used
-  uint32_t qkv[16][3];
+  {
+    uint4 kr[4], qr[4];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int T = c0 + wave * 16 + i;
-    qkv[i][0] = qkv[i][1] = qkv[i][2] = 0u;
-    if (T < p.tokens) {
-      const uint16_t* row = p.mixed + (size_t)T * p.ld_mixed;
-      qkv[i][0] = *reinterpret_cast<const uint32_t*>(row + qoff + 2 * lane);
-      qkv[i][1] = *reinterpret_cast<const uint32_t*>(row + koff + 2 * lane);
-      qkv[i][2] = *reinterpret_cast<const uint32_t*>(row + voff + 2 * lane);
+    for (int i = 0; i < 4; ++i) {
+      const int t = i * 16 + (tid >> 4);
+      const uint16_t* row = p.mixed + (size_t)min(c0 + t, p.tokens - 1) * p.ld_mixed + kh * kDk + (tid & 15) * 8;
+      qr[i] = load16u(row, aligned);
+      kr[i] = load16u(row + key_dim, aligned);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = i * 16 + (tid >> 4), at = t * 16 + ((tid & 15) ^ (t & 15));
+      L.q[at] = qr[i];
+      L.k[at] = kr[i];
     }
   }
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int t = wave * 16 + i;
-    float q0 = 0.f, q1 = 0.f, k0 = 0.f, k1 = 0.f, v0 = 0.f, v1 = 0.f;
-    {
-      const uint32_t qw = qkv[i][0], kw = qkv[i][1], vw = qkv[i][2];
-      q0 = __uint_as_float(qw << 16);
-      q1 = __uint_as_float(qw & 0xFFFF0000u);
-      k0 = __uint_as_float(kw << 16);
-      k1 = __uint_as_float(kw & 0xFFFF0000u);
-      v0 = __uint_as_float(vw << 16);
-      v1 = __uint_as_float(vw & 0xFFFF0000u);
-    }
-    const float rq = 1.0f / sqrtf(wave_sum(q0 * q0 + q1 * q1) + 1e-6f);
-    const float rk = 1.0f / sqrtf(wave_sum(k0 * k0 + k1 * k1) + 1e-6f);
-    L.Q[t][2 * lane] = (q0 * rq) / qscale;
-    L.Q[t][2 * lane + 1] = (q1 * rq) / qscale;
-    L.K[t][2 * lane] = k0 * rk;
-    L.K[t][2 * lane + 1] = k1 * rk;
-    L.V[t][2 * lane] = v0;
-    L.V[t][2 * lane + 1] = v1;
-  }
+  float gam = 0.0f;
   if (wave == 0) {
     const int T = c0 + lane;
-    float g = 0.0f, beta = 0.0f;
+    float beta = 0.0f;
     if (T < p.tokens) {
       const float av = bf2f(p.a[(size_t)T * p.ld_ab + h]), bv = bf2f(p.b[(size_t)T * p.ld_ab + h]);
-      beta = round_bf(sigmoid(bv));                                          // bf16 sigmoid
-      g = -expf(bf2f(p.A_log[h])) * softplus(av + bf2f(p.dt_bias[h]));      // fp32 (reference.py:528-532)
+      beta = round_bf(sigmoid(bv));                                         // bf16 sigmoid
+      gam = -expf(bf2f(p.A_log[h])) * softplus(av + bf2f(p.dt_bias[h]));   // fp32 (reference.py:528-532)
     }
-    float gam = g;  // inclusive prefix sum over the chunk
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
+    for (int off = 1; off < 64; off <<= 1) {  // inclusive prefix sum over the chunk
       const float o = __shfl_up(gam, off, 64);
       if (lane >= off) gam += o;
     }
-    const float last = readlane(gam, 63);
     L.gam[lane] = gam;
     L.beta[lane] = beta;
-    L.eg[lane] = expf(gam);
-    L.dec[lane] = expf(last - gam);
-    if (lane == 0) scratch[(size_t)gridDim.x * p.num_v_heads * kPrepMats * kMat + (size_t)chunk * p.num_v_heads + h] =
-        expf(last);
   }
   __syncthreads();
 
-  // ---- A' and QK (4 x 4 register tiles of the lower triangle) ---------------------------
-  // The 136 tiles (tb, jb <= tb) go to threads p = 4 lane + wave < 136, spread evenly over
-  // the waves; the other threads write the zero tiles above the diagonal.
+  // lane: rows 16 wave + 4 q4 + r, column 16 c + n16 of block (wave, c)
+  auto operand = [&](const uint4* m, int blk, int s) { return m[(blk * 16 + n16) * 16 + ((4 * s + q4) ^ n16)]; };
+  df_f32x4 kk[4], qk[4], qq = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < 4; ++c) kk[c] = qk[c] = df_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const uint4 ka = operand(L.k, wave, s), qa = operand(L.q, wave, s);
+    qq = mfma(qa, qa, qq);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (c <= wave) {
+        const uint4 kb = operand(L.k, c, s);
+        kk[c] = mfma(ka, kb, kk[c]);
+        qk[c] = mfma(qa, kb, qk[c]);
+      }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (4 * q4 + r == n16) {
+      float dk = 0.0f;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (c == wave) dk = kk[c][r];
+      L.nk[16 * wave + n16] = 1.0f / sqrtf(dk + 1e-6f);
+      L.nq[16 * wave + n16] = 1.0f / sqrtf(qq[r] + 1e-6f) / sqrtf(static_cast<float>(kDk));
+    }
+  __syncthreads();
+  float gt[4], bt[4], nkt[4], nqt[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int t = 16 * wave + 4 * q4 + r;
+    gt[r] = L.gam[t], bt[r] = L.beta[t], nkt[r] = L.nk[t], nqt[r] = L.nq[t];
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    if (c <= wave) {
+      const int j = 16 * c + n16;
+      const float gj = L.gam[j], nj = L.nk[j];
+      float* qout = base + kPrepQk + tri(wave, c) * kBlk + (n16 >> 2) * 64 + (n16 & 3);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = 16 * wave + 4 * q4 + r;
+        const float d = j <= t ? expf(gt[r] - gj) * nj : 0.0f;
+        L.a[tri(wave, c)][4 * q4 + r][n16] = j < t ? bt[r] * (kk[c][r] * nkt[r] * d) : 0.0f;
+        qout[(4 * q4 + r) * 4] = qk[c][r] * nqt[r] * d;
+      }
+    }
+  if (wave == 0) {
+    const float last = readlane(gam, 63), eg = expf(gam), nk = L.nk[lane];
+    base[kPrepTok + lane] = L.beta[lane] * eg * nk;
+    base[kPrepTok + kCk + lane] = L.beta[lane];
+    base[kPrepTok + 2 * kCk + lane] = expf(last - gam) * nk;
+    base[kPrepTok + 3 * kCk + lane] = eg * L.nq[lane];
+    if (lane < 16) base[kPrepEc + lane] = expf(last);
+  }
+  // the wave's own block of A' is complete for the wave: its inverse, column n16 in registers
   {
-    const int pidx = 4 * lane + wave;
-    int tb, jb;
-    if (pidx < 136) {
-      tb = 0;
-      while ((tb + 1) * (tb + 2) / 2 <= pidx) ++tb;
-      jb = pidx - tb * (tb + 1) / 2;
-    } else {  // upper tiles: 120 of them, for the 120 threads 136 .. 255
-      const int q = pidx - 136;  // (jb, tb) with tb < jb
-      jb = 1;
-      while (jb * (jb + 1) / 2 <= q) ++jb;
-      tb = q - jb * (jb - 1) / 2;
-    }
-    float aa[4][4], qq[4][4];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const int d = tri(wave, wave);
+    float x[16];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int t = 0; t < 16; ++t) x[t] = t == n16 ? 1.0f : 0.0f;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) aa[r][c] = qq[r][c] = 0.0f;
-    if (jb <= tb) {
-      for (int k = 0; k < kDk; k += 4) {
-        float4 kt[4], kj[4], qt[4];
+    for (int t = 1; t < 16; ++t) {
+      float row[16];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          kt[r] = *reinterpret_cast<const float4*>(&L.K[tb * 4 + r][k]);
-          qt[r] = *reinterpret_cast<const float4*>(&L.Q[tb * 4 + r][k]);
-          kj[r] = *reinterpret_cast<const float4*>(&L.K[jb * 4 + r][k]);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            aa[r][c] += kt[r].x * kj[c].x + kt[r].y * kj[c].y + kt[r].z * kj[c].z + kt[r].w * kj[c].w;
-            qq[r][c] += qt[r].x * kj[c].x + qt[r].y * kj[c].y + qt[r].z * kj[c].z + qt[r].w * kj[c].w;
-          }
+      for (int j = 0; j < t; j += 4) {
+        const float4 v = *reinterpret_cast<const float4*>(&L.a[d][t][j]);
+        row[j] = v.x, row[j + 1] = v.y, row[j + 2] = v.z, row[j + 3] = v.w;
       }
+#pragma unroll
+      for (int j = 0; j < t; ++j) x[t] = fmaf(-row[j], x[j], x[t]);
     }
+    if (q4 == 0) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+      for (int t = 0; t < 16; t += 4)
+        *reinterpret_cast<float4*>(&L.tt[d][n16][t]) = make_float4(x[t], x[t + 1], x[t + 2], x[t + 3]);
+    }
+    if (q4 == 1) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int t = tb * 4 + r, j = jb * 4 + c;
-        const float d = j <= t ? expf(L.gam[t] - L.gam[j]) : 0.0f;
-        L.At[j][t] = j < t ? L.beta[t] * (aa[r][c] * d) : 0.0f;
-        L.QK[t][j] = j <= t ? qq[r][c] * d : 0.0f;
-      }
-  }
-  float* base = scratch + prep_base(chunk, h, p.num_v_heads);
-  // Kd = diag(exp(gamma_C - gamma)) K, before K becomes a right-hand side
-  for (int e = tid; e < kMat; e += 256) base[4 * kMat + e] = L.dec[e / kDk] * L.K[e / kDk][e % kDk];
-  __syncthreads();
-  for (int e = tid; e < kMat; e += 256) {
-    const int t = e / kDk, k = e % kDk;
-    L.V[t][k] *= L.beta[t];
-    L.K[t][k] *= L.beta[t] * L.eg[t];
+      for (int t = 0; t < 16; ++t) L.td[wave][t][n16] = x[t];
+    }
   }
   __syncthreads();
+#pragma unroll
+  for (int dist = 1; dist < 4; ++dist) {
+    if (wave >= dist) {
+      const int b = wave, a = wave - dist;
+      df_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < dist; ++i) {
+        const int c = a + i;
+        acc = mfma16(*reinterpret_cast<const float4*>(&L.a[tri(b, c)][n16][4 * q4]),
+                     *reinterpret_cast<const float4*>(&L.tt[tri(c, a)][n16][4 * q4]), acc);
+      }
+      *reinterpret_cast<float4*>(&L.pt[wave - 1][n16][4 * q4]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      df_f32x4 t = {0.f, 0.f, 0.f, 0.f};
+      t = mfma16(*reinterpret_cast<const float4*>(&L.td[b][n16][4 * q4]),
+                 *reinterpret_cast<const float4*>(&L.pt[wave - 1][n16][4 * q4]), t);
+      *reinterpret_cast<float4*>(&L.tt[tri(b, a)][n16][4 * q4]) = make_float4(-t[0], -t[1], -t[2], -t[3]);
+    }
+    __syncthreads();
+  }
+  // T out: float (j / 4, t, j % 4) of a block from its transposed [j][t]
+#pragma unroll
+  for (int i = 0; i < kTri; ++i)
+    base[i * kBlk + tid] = L.tt[i][(tid >> 6) * 4 + (tid & 3)][(tid >> 2) & 15];
+}
 
-  // ---- forward substitution: X_t = R_t - sum_{j<t} A'[t][j] X_j, in place --------------
-  // Lane = one of the 256 columns of [V | K] (wave w: columns 64 w ..), its 64 tokens in
-  // registers. Once token t is final, t's multiple is taken off every later token u, with
-  // A'[u][t] read from row t of At as uniform LDS broadcasts. Each token receives its terms in
-  // the order j = 0, 1, .. with the same fmaf as a token-by-token solve, but every step's
-  // updates are independent of each other.
-  {
-    float (*M)[kPitch] = wave < 2 ? L.V : L.K;
-    const int col = (wave & 1) * 64 + lane;
-    float x[kCk];
+// Two fp32 as three bf16 each, whose sums they are: 8 significant bits apiece, every remainder
+// exact. Component i holds both values' part i, packed.
+DF_DEVICE void split3(float a, float b, uint32_t (&part)[3]) {
 #pragma unroll
-    for (int t = 0; t < kCk; ++t) x[t] = M[t][col];
-#pragma unroll
-    for (int t = 0; t < kCk - 1; ++t) {
-#pragma unroll
-      for (int u4 = (t + 1) & ~3; u4 < kCk; u4 += 4) {
-        const float4 a = *reinterpret_cast<const float4*>(&L.At[t][u4]);
-        const float av[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (u4 + e > t) x[u4 + e] = fmaf(-av[e], x[t], x[u4 + e]);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < kCk; ++t) M[t][col] = x[t];
-  }
-  __syncthreads();
-
-  // ---- O_loc = QK Wv and Qx = diag(e^gamma) Q - QK Wk; Wv, Wk out ----------------------
-  {
-    // token t = 4 (li % 16) + wave for li = tid / 4: each wave gets every fourth token, so the
-    // triangular work (t + 1 terms) is spread evenly
-    const int li = tid >> 2, t = 4 * (li & 15) + wave, cs = (tid & 3) * 32;
-    float o[32], qx[32];
-#pragma unroll
-    for (int c = 0; c < 32; ++c) {
-      o[c] = 0.0f;
-      qx[c] = 0.0f;
-    }
-    for (int j = 0; j <= t; ++j) {
-      const float w = L.QK[t][j];
-#pragma unroll
-      for (int c = 0; c < 32; c += 4) {
-        const float4 wv = *reinterpret_cast<const float4*>(&L.V[j][cs + c]);
-        const float4 wk = *reinterpret_cast<const float4*>(&L.K[j][cs + c]);
-        o[c] += w * wv.x; o[c + 1] += w * wv.y; o[c + 2] += w * wv.z; o[c + 3] += w * wv.w;
-        qx[c] += w * wk.x; qx[c + 1] += w * wk.y; qx[c + 2] += w * wk.z; qx[c + 3] += w * wk.w;
-      }
-    }
-    const float egt = L.eg[t];
-    float* orow = base + (size_t)t * kDk + cs;
-    float* qrow = base + kMat + (size_t)t * kDk + cs;
-#pragma unroll
-    for (int c = 0; c < 32; c += 4) {
-      *reinterpret_cast<float4*>(orow + c) = make_float4(o[c], o[c + 1], o[c + 2], o[c + 3]);
-      *reinterpret_cast<float4*>(qrow + c) =
-          make_float4(egt * L.Q[t][cs + c] - qx[c], egt * L.Q[t][cs + c + 1] - qx[c + 1],
-                      egt * L.Q[t][cs + c + 2] - qx[c + 2], egt * L.Q[t][cs + c + 3] - qx[c + 3]);
-    }
-  }
-  for (int e = tid; e < kMat; e += 256) {
-    base[2 * kMat + e] = L.V[e / kDk][e % kDk];
-    base[3 * kMat + e] = L.K[e / kDk][e % kDk];
+  for (int i = 0; i < 3; ++i) {
+    part[i] = pack_bf16(a, b);
+    a -= __uint_as_float(part[i] << 16);
+    b -= __uint_as_float(part[i] & 0xFFFF0000u);
   }
 }
 
-// The scan: one workgroup per (value head, 16 value columns), the chunks in order. Per chunk:
-// O = O_loc + Qx S0 (tokens out as bf16), delta = Wv - Wk S0, S = e^gamma_C S0 + Kd^T delta,
-// all on the fp32 MFMA (v_mfma_f32_16x16x4_f32):
-// - O and delta: wave w owns tokens 16 w ..+15 (16 x 16 results over k = 128). Its A operands
-//   (rows of Qx and Wk) come straight from the pre-pass scratch; B is S, shared through LDS
-//   transposed (St[c][k]);
-// - the update: wave w owns state rows k = 32 w ..+31 (two 16 x 16 tiles over the 64 tokens),
-//   kept in registers in the MFMA result layout. A is Kd^T, read from the scratch; B is
-//   delta, shared through LDS transposed (Dt[c][t]).
-// Each lane takes k (or t) in runs of 4 (k = 16 s + 4 (lane / 16) + j for the MFMA j of
-// group s), so its operands are 16-byte loads. Every global operand of the next chunk is
-// loaded a chunk ahead (two register sets).
+// The scan: one workgroup per (value head, 16 value columns), eight waves, the chunks in order.
+// Wave w holds state rows 16 w .. + 15 in the product's result layout; S0 lies in LDS as
+// three bf16 planes, transposed. Per chunk, a barrier after each:
+//   1. waves 0..3 (16 tokens each): Y = K S0 and Z = Q S0 from one read of the planes,
+//      R = beta V - (beta e^gamma rk) Y and Z into LDS;
+//      waves 4..7: the next chunk's K rows by global_load_lds, this chunk's QK blocks into
+//      registers, and the outputs of the chunk before, O = (e^gamma rq / sqrt(Dk)) Z + QK delta;
+//   2. waves 0..3: delta = T R, into LDS in fp32 and, times exp(gamma_C - gamma) rk, in three planes;
+//   3. every wave: S = e^gamma_C S + K^T delta (K read transposed by ds_read_tr16_b64), its planes.
+// Every operand that is a lane's own is loaded a chunk ahead into registers.
+// A serial chain of three steps a chunk, 2.5 us: 256 workgroups for 32 heads are one per CU, so
+// wider column tiles would idle CUs. Without any loads the loop takes about 95 of
+// the 157 us (4096 tokens, 32 heads), without T R too about 75. 319 us with the rows in fp32
+// and every product on the fp32 unit. The T, Q and V loads are issued after step 2's products:
+// at the start of step 1 they cost 12 us more, after its products 13.
 constexpr int kScanVs = 16;
+constexpr int kScanThreads = 512;
 
 struct ScanLds {
-  float St[kScanVs][kDk + 4];   // S0 transposed
-  float Dt[kScanVs][kCk + 4];   // delta transposed
+  uint4 k[2][kCk * 16];              // raw K rows, 16-byte chunk c of row t in slot c ^ (t % 16)
+  uint16_t s[3][kScanVs][kDk];       // S0's planes transposed, 16-byte chunk c of column n in slot c ^ n
+  float r[kScanVs][kCk + 4];         // R transposed
+  float d[2][kScanVs][kCk + 4];      // delta transposed, two chunks
+  float4 z[2][4][64];                // Z as the lanes of waves 0..3 hold it, two chunks
+  uint16_t dp[3][kScanVs][kCk + 8];  // the scaled delta's planes, transposed
 };
 
-struct ScanPre {                // one chunk's operands for one lane
-  float4 qa[8], wa[8];          // Qx, Wk: row 16 w + lane % 16, k = 16 s + 4 (lane / 16) ..+3
-  float kd[2][4][4];            // Kd[t = 16 s + 4 (lane / 16) + j][k = 32 w + 16 tile + lane % 16]
-  float ol[4], wv[4];           // O_loc, Wv at (16 w + 4 (lane / 16) + r, column lane % 16)
-};
-
-DF_DEVICE df_f32x4 mfma4(float a, float b, df_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
-__global__ __launch_bounds__(256) void delta_scan_kernel(DfDeltaPrefillArgs p, const float* __restrict__ scratch) {
-  __shared__ __align__(16) ScanLds L;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int h = blockIdx.x, vs = blockIdx.y;
-  const int col0 = vs * kScanVs;
+__global__ __launch_bounds__(kScanThreads) void delta_scan_kernel(DfDeltaPrefillArgs p, const float* __restrict__ scratch,
+                                                                  int aligned) {
+  __shared__ __align__(1024) ScanLds L;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = blockIdx.x, hv = p.num_v_heads;
+  const int col0 = blockIdx.y * kScanVs;
   const int nchunks = (p.tokens + kCk - 1) / kCk;
   const int n16 = lane & 15, q4 = lane >> 4;
+  const bool kwave = wave < 4;
+  const int w4 = wave & 3, t4 = 16 * w4 + 4 * q4;  // the wave's token block, the lane's 4 result tokens
+  const int qoff = h / (hv / p.num_k_heads) * kDk, koff = qoff + p.num_k_heads * kDk;
+  const int voff = 2 * p.num_k_heads * kDk + h * kDk + col0 + n16;
   float* gstate = p.state + (size_t)h * kDk * kDk;
-  const float* ecs = scratch + (size_t)nchunks * p.num_v_heads * kPrepMats * kMat;
+  const uint32_t lds_k = lds_offset(&L.k[0][0]);
 
-  // this wave's state rows in the MFMA result layout: S[32 w + 16 tile + 4 q4 + r][n16]
-  df_f32x4 S[2];
+  df_f32x4 S;  // rows 16 wave + 4 q4 + r, column n16
 #pragma unroll
-  for (int tl = 0; tl < 2; ++tl)
+  for (int r = 0; r < 4; ++r) S[r] = gstate[(size_t)(16 * wave + 4 * q4 + r) * kDk + col0 + n16];
+  auto put4 = [&](uint16_t* plane, int stride, float v0, float v1, float v2, float v3) {  // into the three planes
+    uint32_t a[3], b[3];
+    split3(v0, v1, a);
+    split3(v2, v3, b);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) S[tl][r] = gstate[(size_t)(32 * wave + 16 * tl + 4 * q4 + r) * kDk + col0 + n16];
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2*>(plane + i * stride) = make_uint2(a[i], b[i]);
+  };
   auto put_state = [&]() {
-#pragma unroll
-    for (int tl = 0; tl < 2; ++tl)
-      *reinterpret_cast<float4*>(&L.St[n16][32 * wave + 16 * tl + 4 * q4]) = make_float4(S[tl][0], S[tl][1], S[tl][2], S[tl][3]);
+    const int k = 16 * wave + 4 * q4;
+    put4(&L.s[0][n16][((k >> 3) ^ n16) * 8 + (k & 7)], kScanVs * kDk, S[0], S[1], S[2], S[3]);
   };
-  auto fetch = [&](ScanPre& P, int chunk) {
-    const float* base = scratch + prep_base(chunk, h, p.num_v_heads);
-    const int row = 16 * wave + n16;
+
+  // K rows of a chunk, by waves 4..7: rows i * 16 + (tid - 256) / 16, slot tid % 16
+  auto issue_k = [&](int chunk) {
+    const int at = chunk * kCk, last = p.tokens - 1 - at;
+    const uint16_t* rows = p.mixed + (size_t)at * p.ld_mixed + koff;
 #pragma unroll
-    for (int sg = 0; sg < 8; ++sg) {
-      P.qa[sg] = *reinterpret_cast<const float4*>(base + kMat + (size_t)row * kDk + 16 * sg + 4 * q4);
-      P.wa[sg] = *reinterpret_cast<const float4*>(base + 3 * kMat + (size_t)row * kDk + 16 * sg + 4 * q4);
+    for (int i = 0; i < 4; ++i) {
+      const int row = i * 16 + ((tid >> 4) & 15), c = (tid & 15) ^ (row & 15);
+      const uint16_t* src = rows + (size_t)min(row, last) * p.ld_mixed + c * 8;
+      if (aligned)
+        dma16(src, lds_k + (chunk & 1) * (kCk * 256) + w4 * 1024 + i * 4096);
+      else
+        L.k[chunk & 1][i * 256 + (tid & 255)] = load16u(src, false);
     }
+  };
+  // A lane's operands of a chunk. Waves 0..3: T blocks (w4, c <= w4), the factors beta e^gamma rk,
+  // beta and exp(gamma_C - gamma) rk at tokens t4 .. + 3, V there, and Q's row 16 w4 + n16, dims
+  // 32 s + 8 q4 ..+7.
+  struct Ops {
+    float4 t[4], f0, f1, f2;
+    uint32_t v[4];
+    uint4 q[4];
+  };
+  const size_t v_at = (size_t)t4 * p.ld_mixed + voff, q_at = (size_t)(16 * w4 + n16) * p.ld_mixed + qoff + q4 * 8;
+  auto fetch = [&](int chunk) {
+    Ops o;
+    const float* base = scratch + prep_base(chunk, h, hv);
+    const float* blk = base + tri(w4, 0) * kBlk + lane * 4;
 #pragma unroll
-    for (int tl = 0; tl < 2; ++tl)
+    for (int c = 0; c < 4; ++c) o.t[c] = *reinterpret_cast<const float4*>(blk + min(c, w4) * kBlk);
+    const float* tok = base + kPrepTok + t4;
+    o.f0 = *reinterpret_cast<const float4*>(tok);
+    o.f1 = *reinterpret_cast<const float4*>(tok + kCk);
+    o.f2 = *reinterpret_cast<const float4*>(tok + 2 * kCk);
+    const int at = chunk * kCk, last = p.tokens - 1 - at;
+    const uint16_t* rows = p.mixed + (size_t)at * p.ld_mixed;
+    if (last >= kCk - 1) {  // a full chunk: uniform bases and the lane's offsets, no address arithmetic
 #pragma unroll
-      for (int sg = 0; sg < 4; ++sg)
+      for (int r = 0; r < 4; ++r) o.v[r] = rows[(size_t)r * p.ld_mixed + v_at];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          P.kd[tl][sg][j] = base[4 * kMat + (size_t)(16 * sg + 4 * q4 + j) * kDk + 32 * wave + 16 * tl + n16];
+      for (int s = 0; s < 4; ++s) o.q[s] = load16u(rows + s * 32 + q_at, aligned);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o.v[r] = rows[(size_t)min(t4 + r, last) * p.ld_mixed + voff];
+      const uint16_t* row = rows + (size_t)min(16 * w4 + n16, last) * p.ld_mixed + qoff + q4 * 8;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) o.q[s] = load16u(row + s * 32, aligned);
+    }
+    return o;
+  };
+  // Waves 4..7: QK blocks (w4, c <= w4) and the factor e^gamma rq / sqrt(Dk) at tokens t4 .. + 3.
+  struct Outs {
+    float4 qk[4], f;
+  };
+  auto fetch_out = [&](int chunk) {
+    Outs o;
+    const float* base = scratch + prep_base(chunk, h, hv);
+    const float* blk = base + kPrepQk + tri(w4, 0) * kBlk + lane * 4;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o.qk[c] = *reinterpret_cast<const float4*>(blk + min(c, w4) * kBlk);
+    o.f = *reinterpret_cast<const float4*>(base + kPrepTok + 3 * kCk + t4);
+    return o;
+  };
+  auto outputs = [&](const Outs& o, int chunk) {
+    df_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (c <= w4)
+        acc = mfma16(o.qk[c], *reinterpret_cast<const float4*>(&L.d[chunk & 1][n16][16 * c + 4 * q4]), acc);
+    const float4 z = L.z[chunk & 1][w4][lane];
+    const float v[4] = {fmaf(o.f.x, z.x, acc[0]), fmaf(o.f.y, z.y, acc[1]), fmaf(o.f.z, z.z, acc[2]),
+                        fmaf(o.f.w, z.w, acc[3])};
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const size_t e = (size_t)(16 * wave + 4 * q4 + r) * kDk + col0 + n16;
-      P.ol[r] = base[e];
-      P.wv[r] = base[2 * kMat + e];
+      const int T = chunk * kCk + t4 + r;
+      if (T < p.tokens) p.out[(size_t)T * p.ld_out + h * kDk + col0 + n16] = f2bf(v[r]);
     }
   };
-  auto step = [&](const ScanPre& P, ScanPre& N, int chunk) {
-    __syncthreads();  // St holds this chunk's S0
-    if (chunk + 1 < nchunks) fetch(N, chunk + 1);
-    // O and delta for tokens 16 w + 4 q4 + r, column n16
-    df_f32x4 o = {P.ol[0], P.ol[1], P.ol[2], P.ol[3]}, d = {P.wv[0], P.wv[1], P.wv[2], P.wv[3]};
-    df_f32x4 qs = {0.f, 0.f, 0.f, 0.f}, ws = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int sg = 0; sg < 8; ++sg) {
-      const float4 b = *reinterpret_cast<const float4*>(&L.St[n16][16 * sg + 4 * q4]);
-      qs = mfma4(P.qa[sg].x, b.x, qs);
-      qs = mfma4(P.qa[sg].y, b.y, qs);
-      qs = mfma4(P.qa[sg].z, b.z, qs);
-      qs = mfma4(P.qa[sg].w, b.w, qs);
-      ws = mfma4(P.wa[sg].x, b.x, ws);
-      ws = mfma4(P.wa[sg].y, b.y, ws);
-      ws = mfma4(P.wa[sg].z, b.z, ws);
-      ws = mfma4(P.wa[sg].w, b.w, ws);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      o[r] += qs[r];
-      d[r] -= ws[r];
-      const int T = chunk * kCk + 16 * wave + 4 * q4 + r;
-      if (T < p.tokens) p.out[(size_t)T * p.ld_out + h * kDk + col0 + n16] = f2bf(o[r]);
-    }
-    *reinterpret_cast<float4*>(&L.Dt[n16][16 * wave + 4 * q4]) = make_float4(d[0], d[1], d[2], d[3]);
-    __syncthreads();  // Dt complete; every wave is done reading St
-    // S <- e^gamma_C S0 + Kd^T delta
-    const float ec = ecs[(size_t)chunk * p.num_v_heads + h];
-#pragma unroll
-    for (int tl = 0; tl < 2; ++tl) {
-      df_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int sg = 0; sg < 4; ++sg) {
-        const float4 b = *reinterpret_cast<const float4*>(&L.Dt[n16][16 * sg + 4 * q4]);
-        acc = mfma4(P.kd[tl][sg][0], b.x, acc);
-        acc = mfma4(P.kd[tl][sg][1], b.y, acc);
-        acc = mfma4(P.kd[tl][sg][2], b.z, acc);
-        acc = mfma4(P.kd[tl][sg][3], b.w, acc);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S[tl][r] = ec * S[tl][r] + acc[r];
-    }
-    put_state();
-  };
+
   put_state();
-  ScanPre A, B;
-  fetch(A, 0);
-  for (int chunk = 0; chunk < nchunks; chunk += 2) {
-    step(A, B, chunk);
-    if (chunk + 1 < nchunks) step(B, A, chunk + 1);
+  const float* ecp = scratch + kPrepEc + (lane & 15);
+  float ec_next = ecp[prep_base(0, h, hv)];
+  Ops next;
+  Outs out;
+  if (kwave)
+    next = fetch(0);
+  else
+    issue_k(0);
+  for (int chunk = 0; chunk < nchunks; ++chunk) {
+    wait_vm<0>();     // this wave's operands and K rows have arrived
+    __syncthreads();  // every wave's K rows and S0's planes are in LDS
+    const float ec = ec_next;
+    const int ahead = min(chunk + 1, nchunks - 1);
+    Ops cur;
+    // ---- 1: Y, Z and R; the outputs of the chunk before
+    if (kwave) {
+      cur = next;
+      df_f32x4 y[3], z[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) y[i] = z[i] = df_f32x4{0.f, 0.f, 0.f, 0.f};
+      const uint4* kt = &L.k[chunk & 1][(16 * w4 + n16) * 16];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int slot = (4 * s + q4) ^ n16;
+        const uint4 ka = kt[slot];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const uint4 b = *reinterpret_cast<const uint4*>(&L.s[i][n16][slot * 8]);
+          y[i] = mfma(ka, b, y[i]);
+          z[i] = mfma(cur.q[s], b, z[i]);
+        }
+      }
+      const df_f32x4 ys = y[0] + (y[1] + y[2]), zs = z[0] + (z[1] + z[2]);  // smallest first
+      *reinterpret_cast<float4*>(&L.r[n16][t4]) = make_float4(fmaf(-cur.f0.x, ys[0], cur.f1.x * bf2f(cur.v[0])),
+                                                              fmaf(-cur.f0.y, ys[1], cur.f1.y * bf2f(cur.v[1])),
+                                                              fmaf(-cur.f0.z, ys[2], cur.f1.z * bf2f(cur.v[2])),
+                                                              fmaf(-cur.f0.w, ys[3], cur.f1.w * bf2f(cur.v[3])));
+      L.z[chunk & 1][w4][lane] = make_float4(zs[0], zs[1], zs[2], zs[3]);
+    } else {
+      if (chunk + 1 < nchunks) issue_k(chunk + 1);
+      const Outs mine = out;
+      out = fetch_out(chunk);
+      if (chunk > 0) outputs(mine, chunk - 1);  // its stores last: nothing waits for them
+    }
+    __syncthreads();
+    // ---- 2: delta
+    ec_next = ecp[prep_base(ahead, h, hv)];
+    if (kwave) {
+      df_f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (c <= w4) d = mfma16(cur.t[c], *reinterpret_cast<const float4*>(&L.r[n16][16 * c + 4 * q4]), d);
+      next = fetch(ahead);  // issued while the products run
+      *reinterpret_cast<float4*>(&L.d[chunk & 1][n16][t4]) = make_float4(d[0], d[1], d[2], d[3]);
+      put4(&L.dp[0][n16][t4], kScanVs * (kCk + 8), d[0] * cur.f2.x, d[1] * cur.f2.y, d[2] * cur.f2.z, d[3] * cur.f2.w);
+    }
+    __syncthreads();
+    // ---- 3: the state
+    df_f32x4 add[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) add[i] = df_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      // K^T: dims 16 wave + n16, tokens 32 s + 8 q4 ..+7 (two transposed reads of 4 tokens x 16 dims)
+      uint2 a[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int t = 32 * s + 8 * q4 + 4 * i + (n16 >> 2), c = 2 * wave + ((n16 & 3) >> 1);
+        const uint32_t at = t * 256 + ((c ^ (t & 15)) << 4) + (n16 & 1) * 8;
+        a[i] = __builtin_bit_cast(uint2, read_tr(lds_k + (chunk & 1) * (kCk * 256) + at));
+      }
+      const uint4 av = make_uint4(a[0].x, a[0].y, a[1].x, a[1].y);
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        add[i] = mfma(av, *reinterpret_cast<const uint4*>(&L.dp[i][n16][32 * s + 8 * q4]), add[i]);
+    }
+    const df_f32x4 sum = add[0] + (add[1] + add[2]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[r] = fmaf(ec, S[r], sum[r]);
+    put_state();
   }
+  if (!kwave) outputs(out, nchunks - 1);
 #pragma unroll
-  for (int tl = 0; tl < 2; ++tl)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) gstate[(size_t)(32 * wave + 16 * tl + 4 * q4 + r) * kDk + col0 + n16] = S[tl][r];
+  for (int r = 0; r < 4; ++r) gstate[(size_t)(16 * wave + 4 * q4 + r) * kDk + col0 + n16] = S[r];
 }
 
 // ---------------------------------------------------------------------------------------
@@ -920,11 +1028,6 @@ constexpr int kAtPow2Scale = 1;  // scale is a positive power of two: bf16(s * s
 constexpr int kAtVecGate = 2;    // gate rows allow 8-byte loads
 constexpr int kAtVecOut = 4;     // out rows allow 8-byte stores
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-DF_DEVICE s16x4 read_tr(uint32_t at) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(at));
-}
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 
@@ -1296,7 +1399,7 @@ int df_causal_conv_prefill(const uint16_t* x, int ldx, int tokens, int channels,
 size_t df_delta_rule_prefill_workspace_bytes(int tokens, int num_v_heads) {
   if (tokens < 1 || num_v_heads < 1) return 0;
   const size_t chunks = (size_t)(tokens + kCk - 1) / kCk;
-  return (chunks * num_v_heads * (kPrepMats * (size_t)kMat + 1)) * sizeof(float);
+  return chunks * num_v_heads * kPrepFloats * sizeof(float);
 }
 
 int df_delta_rule_prefill(const DfDeltaPrefillArgs* a, void* workspace, size_t workspace_bytes, hipStream_t stream) {
@@ -1313,9 +1416,10 @@ int df_delta_rule_prefill(const DfDeltaPrefillArgs* a, void* workspace, size_t w
     return DF_WORKSPACE_TOO_SMALL;
   const int chunks = (a->tokens + kCk - 1) / kCk;
   float* scratch = reinterpret_cast<float*>(workspace);
-  hipLaunchKernelGGL(delta_prep_kernel, dim3(chunks, a->num_v_heads), dim3(256), 0, stream, *a, scratch);
-  hipLaunchKernelGGL(delta_scan_kernel, dim3(a->num_v_heads, kDk / kScanVs), dim3(256), 0, stream, *a,
-                     static_cast<const float*>(scratch));
+  const int aligned = aligned16(a->mixed) && a->ld_mixed % 8 == 0;  // rows allow 16-byte loads
+  hipLaunchKernelGGL(delta_prep_kernel, dim3(chunks, a->num_v_heads), dim3(256), 0, stream, *a, scratch, aligned);
+  hipLaunchKernelGGL(delta_scan_kernel, dim3(a->num_v_heads, kDk / kScanVs), dim3(kScanThreads), 0, stream, *a,
+                     static_cast<const float*>(scratch), aligned);
   DF_RETURN_LAUNCH_STATUS();
 }
 

@@ -118,6 +118,8 @@ def delta_rule_prefill(mixed: Tensor, a: Tensor, b: Tensor, A_log: Tensor, dt_bi
     ops._check_dtype(op, "dt_bias", dt_bias, BF16, hv)
     if out is None:
         out = torch.empty((tokens, hv * 128), dtype=BF16, device=mixed.device)
+    elif out.untyped_storage().data_ptr() == mixed.untyped_storage().data_ptr():
+        mixed = mixed.clone()  # the scan reads q, k and v while it writes out
     ops.require_gpus(op, mixed, a, b, A_log, dt_bias, state, out)
     nbytes = int(N.lib().df_delta_rule_prefill_workspace_bytes(tokens, hv))
     ws = ops.workspace(mixed.device, nbytes, "delta_prefill")

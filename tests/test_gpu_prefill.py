@@ -182,6 +182,37 @@ def test_delta_rule_prefill_matches_the_scan(tokens):
     _rel_close(st, want_state, 1e-4, f"delta state P={tokens}")
 
 
+@pytest.mark.parametrize("tokens,hk,hv,shift,pad", [
+    (15, 1, 1, 0, 0), (17, 2, 6, 2, 0), (64, 1, 4, 0, 2), (127, 2, 2, 2, 6), (128, 2, 4, 0, 8), (129, 1, 3, 8, 0),
+    (191, 2, 8, 4, 4)])
+def test_delta_rule_prefill_edges(tokens, hk, hv, shift, pad):
+    """16-token blocks and 64-token chunks with remainders, head ratios, and rows that allow only
+    4-byte loads (``shift`` and ``pad`` elements before and after each); an ``out`` inside ``mixed``'s
+    own memory; and the same bits when the tokens come in two calls split at a chunk."""
+    print(f"delta prefill edges {tokens} {hk} {hv} {shift} {pad}", flush=True)
+    mixed, ab, A_log, dt_bias, state = _delta_case(tokens, seed=tokens, hk=hk, hv=hv)
+    width = mixed.shape[1]
+    wide = torch.zeros((tokens, width + shift + pad), dtype=torch.bfloat16, device=DEV)[:, shift:shift + width]
+    wide.copy_(mixed)
+    ab_d, al, dt = ab.to(DEV), A_log.to(DEV), dt_bias.to(DEV)
+
+    def run(at, end, st, **kw):
+        return delta_rule_prefill(wide[at:end], ab_d[at:end, :hv], ab_d[at:end, hv:], al, dt, st, num_k_heads=hk, **kw)
+
+    st = state.to(DEV)
+    got = run(0, tokens, st)
+    want, want_state = _delta_oracle(mixed, ab, A_log, dt_bias, state, hk, hv)
+    close(got, want, what=f"delta out P={tokens}", flip_frac=1e-3)
+    _rel_close(st, want_state, 1e-4, f"delta state P={tokens}")
+    if tokens > 64:
+        st2 = state.to(DEV)
+        parts = torch.cat([run(0, 64, st2), run(64, tokens, st2)])
+        assert torch.equal(parts, got) and torch.equal(st2, st), "two calls"
+    if (width + shift + pad) % 4 == 0 and shift % 4 == 0:
+        st3 = state.to(DEV)
+        assert torch.equal(run(0, tokens, st3, out=wide[:, :hv * 128]), got), "out within mixed"
+
+
 def test_gated_rms_norm_rows():
     gen = torch.Generator().manual_seed(9)
     tokens, heads = 70, 32
