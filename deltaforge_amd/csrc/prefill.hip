@@ -110,11 +110,27 @@ DF_DEVICE void dma4(const void* gaddr, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(gaddr), "s"(lds_base)
                : "memory", "m0");
 }
-// x / (1 + e^-x) from the hardware's exp2 and reciprocal instead of expf and an IEEE division:
-// 5 VALU instead of about 40. Relative error about 6e-8 (2 + |x|), against the 2e-3 of the bf16
-// rounding that follows; the expf form took 6 us of a 128 x 256 tile's 40.
-DF_DEVICE float silu_fast(float x) {
-  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * x));
+// y[i] = x / (1 + e^-x) of N values from the hardware's exp2 and a reciprocal with one Newton step
+// instead of expf and an IEEE division: 8 VALU instead of about 40. Far out, where the quotient
+// nears fp32's smallest numbers, it is silu() (one branch for the N: one for each took 10 us of
+// the 717 x 2560 x 18432 SwiGLU product's 82). Of the 65536 bf16 inputs every one gives the same
+// bf16 as silu(). With silu() the SwiGLU epilogue takes 6 us more of a 128 x 256 tile's 40, the conv
+// 17 more of 25 (4096 tokens, 8192 channels).
+template <int N>
+DF_DEVICE void silu_fast(const float (&x)[N], float (&y)[N]) {
+  float low = x[0];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float d = 1.0f + __builtin_amdgcn_exp2f(-1.44269504f * x[i]);
+    const float r = __builtin_amdgcn_rcpf(d);
+    y[i] = x[i] * fmaf(fmaf(-d, r, 1.0f), r, r);
+    low = fminf(low, x[i]);
+  }
+  if (__builtin_expect(low < -80.0f, 0)) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (x[i] < -80.0f) y[i] = silu(x[i]);
+  }
 }
 // The same with the global address as a uniform base plus the lane's offset.
 DF_DEVICE void dma16s(const void* base, uint32_t offset, uint32_t lds_base) {
@@ -362,8 +378,11 @@ __global__ __launch_bounds__(128 * WN, 1) void int4_gemm_kernel(DfInt4GemmArgs p
           const float* g = ep + row * SH::kPitch + (c / 16) * 32 + (c & 15);
           const float* g1 = g + 32 * SH::kPitch;
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            y[e] = round_bf(silu_fast(round_bf(g[e] + g1[e]))) * round_bf(g[16 + e] + g1[16 + e]);
+          for (int e = 0; e < 8; ++e) y[e] = round_bf(g[e] + g1[e]);
+          float act[8];
+          silu_fast(y, act);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[e] = round_bf(act[e]) * round_bf(g[16 + e] + g1[16 + e]);
         } else {
           const float* g = ep + row * SH::kPitch + c;
           const float* g1 = g + 32 * SH::kPitch;
@@ -391,40 +410,91 @@ __global__ __launch_bounds__(128 * WN, 1) void int4_gemm_kernel(DfInt4GemmArgs p
 // out[t][c] = bf16(silu(bf16(sum_j w[c][j] x(p - 3 + j)))) for position p = pos0 + t, taps in
 // order with fp32 sums (the decode step's arithmetic); x(q) is row q - pos0 of the input for
 // q >= pos0, else the history ring (slot q mod 4, zero for positions before the first).
+//
+// A thread walks `per` tokens of V channels with the window in registers, so a row is read
+// 1 + 3 / per times; V = 4 (8-byte loads, four rows in flight) where rows allow it, else 1. The
+// threads of the first tokens also put the last three inputs into the ring, after they have
+// read it. 4096 tokens of 8192 channels, 134 MB, with the ring: 89 + 5 us (a thread to an
+// element, four loads each) -> 30; 717 tokens 14 + 5 -> 9. Walks of 8 and 32 tokens take as long.
+template <int V>
 __global__ __launch_bounds__(256) void conv_seq_kernel(const uint16_t* __restrict__ x, int ldx, int tokens,
                                                        int channels, const uint16_t* __restrict__ w,
-                                                       const uint16_t* __restrict__ ring, int pos0,
-                                                       uint16_t* __restrict__ out, int ldo) {
+                                                       uint16_t* __restrict__ ring, int pos0,
+                                                       uint16_t* __restrict__ out, int ldo, int per) {
 #pragma clang fp contract(off)
-  const int c = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
+  static_assert(V == 1 || V == 4, "one channel or four");
+  const int c = (blockIdx.x * 256 + threadIdx.x) * V;
   if (c >= channels) return;
-  const uint2 wt = *reinterpret_cast<const uint2*>(w + (size_t)c * 4);
-  const float wk[4] = {__uint_as_float(wt.x << 16), __uint_as_float(wt.x & 0xFFFF0000u),
-                       __uint_as_float(wt.y << 16), __uint_as_float(wt.y & 0xFFFF0000u)};
-  float h[4];
+  const int t0 = blockIdx.y * per, t1 = min(t0 + per, tokens);
+  float wk[V][4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int tt = t - 3 + j;
-    h[j] = tt >= 0 ? bf2f(x[(size_t)tt * ldx + c]) : bf2f(ring[(size_t)c * 4 + ((pos0 + tt) & 3)]);
+  for (int v = 0; v < V; ++v) {
+    const uint2 wt = *reinterpret_cast<const uint2*>(w + (size_t)(c + v) * 4);
+    wk[v][0] = __uint_as_float(wt.x << 16), wk[v][1] = __uint_as_float(wt.x & 0xFFFF0000u);
+    wk[v][2] = __uint_as_float(wt.y << 16), wk[v][3] = __uint_as_float(wt.y & 0xFFFF0000u);
   }
-  float acc = h[0] * wk[0];
-  acc = acc + h[1] * wk[1];
-  acc = acc + h[2] * wk[2];
-  acc = acc + h[3] * wk[3];
-  out[(size_t)t * ldo + c] = f2bf(silu(round_bf(acc)));
-}
-
-// The last three inputs into the ring (slot position mod 4), after conv_seq_kernel read it.
-__global__ __launch_bounds__(256) void conv_ring_update_kernel(const uint16_t* __restrict__ x, int ldx, int tokens,
-                                                               int channels, uint16_t* __restrict__ ring, int pos0) {
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= channels) return;
+  auto load = [&](int t, float (&h)[V]) {
+    const uint16_t* src = x + (size_t)t * ldx + c;
+    if constexpr (V == 4) {
+      const uint2 r = *reinterpret_cast<const uint2*>(src);
+      h[0] = __uint_as_float(r.x << 16), h[1] = __uint_as_float(r.x & 0xFFFF0000u);
+      h[2] = __uint_as_float(r.y << 16), h[3] = __uint_as_float(r.y & 0xFFFF0000u);
+    } else {
+      h[0] = bf2f(*src);
+    }
+  };
+  float h[7][V];  // rows t - 3 .. t + 3
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
-    const int t = tokens - 3 + j;
-    if (t >= 0) ring[(size_t)c * 4 + ((pos0 + t) & 3)] = x[(size_t)t * ldx + c];
+    const int t = t0 - 3 + j;
+    if (t >= 0) {
+      load(t, h[j]);
+    } else {
+#pragma unroll
+      for (int v = 0; v < V; ++v) h[j][v] = bf2f(ring[(size_t)(c + v) * 4 + ((pos0 + t) & 3)]);
+    }
+  }
+  for (int t = t0; t < t1; t += 4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load(min(t + i, tokens - 1), h[3 + i]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float s[V], y[V];
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        float acc = h[i][v] * wk[v][0];
+        acc = acc + h[i + 1][v] * wk[v][1];
+        acc = acc + h[i + 2][v] * wk[v][2];
+        acc = acc + h[i + 3][v] * wk[v][3];
+        s[v] = round_bf(acc);
+      }
+      silu_fast(s, y);
+      if (t + i < t1) {
+        uint16_t* dst = out + (size_t)(t + i) * ldo + c;
+        if constexpr (V == 4)
+          *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]));
+        else
+          *dst = f2bf(y[0]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int v = 0; v < V; ++v) h[j][v] = h[j + 4][v];
+  }
+  if (t0 == 0) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int t = tokens - 3 + j;
+      if (t < 0) continue;
+#pragma unroll
+      for (int v = 0; v < V; ++v) ring[(size_t)(c + v) * 4 + ((pos0 + t) & 3)] = x[(size_t)t * ldx + c + v];
+    }
   }
 }
+
+// Tokens a thread walks: long walks read fewer rows twice, short ones fill the chip.
+static int conv_tokens(int tokens) { return tokens >= 2048 ? 16 : 4; }
 
 // ---------------------------------------------------------------------------------------
 // chunked gated delta rule (reference.py:403-461 over a sequence)
@@ -1389,10 +1459,12 @@ int df_causal_conv_prefill(const uint16_t* x, int ldx, int tokens, int channels,
   if (!x || !weight || !ring || !out || tokens < 1 || channels < 1 || ldx < channels || ldo < channels || pos0 < 0 ||
       (reinterpret_cast<uintptr_t>(weight) & 7) || tokens > 65535)
     return DF_BAD_ARGUMENT;
-  const int cb = (channels + 255) / 256;
-  hipLaunchKernelGGL(conv_seq_kernel, dim3(cb, tokens), dim3(256), 0, stream, x, ldx, tokens, channels, weight, ring,
-                     pos0, out, ldo);
-  hipLaunchKernelGGL(conv_ring_update_kernel, dim3(cb), dim3(256), 0, stream, x, ldx, tokens, channels, ring, pos0);
+  const bool vec = channels % 4 == 0 && ldx % 4 == 0 && ldo % 4 == 0 && !(reinterpret_cast<uintptr_t>(x) & 7) &&
+                   !(reinterpret_cast<uintptr_t>(out) & 7);
+  const int per = conv_tokens(tokens);
+  const dim3 grid((channels + (vec ? 1023 : 255)) / (vec ? 1024 : 256), (tokens + per - 1) / per);
+  hipLaunchKernelGGL(vec ? conv_seq_kernel<4> : conv_seq_kernel<1>, grid, dim3(256), 0, stream, x, ldx, tokens, channels,
+                     weight, ring, pos0, out, ldo, per);
   DF_RETURN_LAUNCH_STATUS();
 }
 

@@ -144,6 +144,48 @@ def test_causal_conv_prefill_is_conv1d(tokens, pos0):
     assert torch.equal(got_hist, new_hist[0]), "history ring"
 
 
+@pytest.mark.parametrize("tokens,pos0,channels,shift,pad", [
+    (1, 2, 4, 0, 0), (3, 1, 1028, 0, 4), (4, 7, 1020, 0, 0), (5, 0, 6, 0, 2), (17, 3, 260, 4, 0), (17, 3, 260, 1, 0),
+    (31, 6, 257, 0, 3), (2047, 5, 8, 0, 0), (2048, 0, 12, 0, 0), (2050, 9, 5, 0, 0)])
+def test_causal_conv_prefill_edges(tokens, pos0, channels, shift, pad):
+    """Remainders of the tokens a thread walks and of its four channels, rows that allow only
+    2-byte loads, and the history ring read and written by one call; exact, as both sides take the
+    taps in order in fp32."""
+    print(f"conv edges {tokens} {pos0} {channels} {shift} {pad}", flush=True)
+    gen = torch.Generator().manual_seed(tokens + channels)
+    rand = lambda *s: torch.randn(s, generator=gen).to(torch.bfloat16)
+    w, ring, x = rand(channels, 1, 4), rand(channels, 4), rand(tokens, channels)
+    wide = torch.zeros((tokens, channels + shift + pad), dtype=torch.bfloat16, device=DEV)[:, shift:shift + channels]
+    wide.copy_(x)
+    ring_d = ring.to(DEV)
+    got = causal_conv_prefill(wide, w.reshape(channels, 4).to(DEV), ring_d, pos0=pos0)
+    hist = torch.stack([ring[:, (pos0 - 3 + j) % 4] for j in range(3)], dim=-1)
+    want, new_hist = causal_conv(x.t().unsqueeze(0), hist.unsqueeze(0), w)
+    assert torch.equal(got.cpu(), want[0].t()), "conv output"
+    end = pos0 + tokens
+    kept = torch.stack([ring_d.cpu()[:, (end - 3 + j) % 4] for j in range(3)], dim=-1)
+    assert torch.equal(kept, new_hist[0]), "history ring"
+    if tokens < 4:  # the slots that no token fell on
+        same = [s for s in range(4) if s not in {(pos0 + t) % 4 for t in range(tokens)}]
+        assert torch.equal(ring_d.cpu()[:, same], ring[:, same]), "other slots"
+
+
+def test_conv_silu_rounds_every_bf16_like_64_bits():
+    """One token whose channels are all the finite bf16 numbers, weight 1 on its own tap."""
+    bits = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    x = bits[torch.isfinite(bits.float())]
+    w = torch.zeros((x.numel(), 4), dtype=torch.bfloat16)
+    w[:, 3] = 1
+    ring = torch.zeros((x.numel(), 4), dtype=torch.bfloat16, device=DEV)
+    got = causal_conv_prefill(x.unsqueeze(0).to(DEV), w.to(DEV), ring)[0].cpu()
+    x64 = x.double()
+    want = (x64 / (1 + torch.exp(-x64))).to(torch.bfloat16)
+    # e^-x is past fp32's range below -88.7, where the quotient is under 2e-37 and may be zero
+    far = x64 < -88.7
+    assert torch.equal(got[~far], want[~far])
+    assert float(got[far].double().abs().max()) < 2e-37
+
+
 def _delta_case(tokens, seed, hk=16, hv=32):
     gen = torch.Generator().manual_seed(seed)
     mixed = (torch.randn((tokens, (2 * hk + hv) * 128), generator=gen)).to(torch.bfloat16)
