@@ -553,6 +553,22 @@ DF_DEVICE uint4 load16u(const uint16_t* p, bool aligned) {
   const uint32_t* w = reinterpret_cast<const uint32_t*>(p);
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
+DF_DEVICE void store16u(uint16_t* p, const uint4& v, bool aligned) {
+  if (aligned) {
+    *reinterpret_cast<uint4*>(p) = v;
+    return;
+  }
+  uint32_t* w = reinterpret_cast<uint32_t*>(p);
+  w[0] = v.x, w[1] = v.y, w[2] = v.z, w[3] = v.w;
+}
+DF_DEVICE void unpack8(const uint4& v, float (&x)[8]) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[2 * i] = __uint_as_float(w[i] << 16);
+    x[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
+  }
+}
 
 // Four waves; wave w owns tokens 16 w .. + 15. K K^T and Q K^T on 16 x 16 x 32 products (their
 // diagonals and Q Q^T's give the norms), A' into LDS, then T block by block: each wave inverts
@@ -958,28 +974,41 @@ __global__ __launch_bounds__(kScanThreads) void delta_scan_kernel(DfDeltaPrefill
 }
 
 // ---------------------------------------------------------------------------------------
-// GatedRMSNorm over rows (reference.py:115-121): one wave per (token, value head)
+// GatedRMSNorm over rows (reference.py:115-121)
 // ---------------------------------------------------------------------------------------
 
+// Sixteen lanes to a head, 8 dims each (16-byte accesses where `aligned`, else 4-byte ones), so
+// the sum is four exchanges. 4096 tokens of 32 heads, 101 MB: 38 us (a wave to a head) -> 19.
 __global__ __launch_bounds__(256) void gated_norm_rows_kernel(const uint16_t* __restrict__ x, int ldx,
                                                               const uint16_t* __restrict__ z, int ldz,
                                                               const uint16_t* __restrict__ w, float eps, int tokens,
-                                                              int heads, uint16_t* __restrict__ out, int ldo) {
-  const int lane = threadIdx.x & 63;
-  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (unit >= tokens * heads) return;
-  const int t = unit / heads, hh = unit % heads;
-  const int d = hh * 128 + 2 * lane;
-  const uint32_t xv = *reinterpret_cast<const uint32_t*>(x + (size_t)t * ldx + d);
-  const uint32_t zv = *reinterpret_cast<const uint32_t*>(z + (size_t)t * ldz + d);
-  const uint32_t wv = *reinterpret_cast<const uint32_t*>(w + 2 * lane);
-  const float x0 = __uint_as_float(xv << 16), x1 = __uint_as_float(xv & 0xFFFF0000u);
-  const float r = 1.0f / sqrtf(wave_sum(x0 * x0 + x1 * x1) / 128.0f + eps);
-  const float n0 = round_bf(x0 * r), n1 = round_bf(x1 * r);
-  const float y0 = round_bf(__uint_as_float(wv << 16) * n0), y1 = round_bf(__uint_as_float(wv & 0xFFFF0000u) * n1);
-  const float g0 = silu(__uint_as_float(zv << 16)), g1 = silu(__uint_as_float(zv & 0xFFFF0000u));
-  *reinterpret_cast<uint32_t*>(out + (size_t)t * ldo + d) =
-      static_cast<uint32_t>(f2bf(y0 * g0)) | (static_cast<uint32_t>(f2bf(y1 * g1)) << 16);
+                                                              int heads, uint16_t* __restrict__ out, int ldo,
+                                                              int aligned) {
+  const long unit = (long)blockIdx.x * 16 + (threadIdx.x >> 4);
+  if (unit >= (long)tokens * heads) return;
+  const int t = unit / heads, hh = unit - (long)t * heads;
+  const int d = (threadIdx.x & 15) * 8, at = hh * 128 + d;
+  float xv[8], zv[8], wv[8];
+  unpack8(load16u(x + (size_t)t * ldx + at, aligned), xv);
+  unpack8(load16u(z + (size_t)t * ldz + at, aligned), zv);
+  unpack8(load16u(w + d, aligned), wv);
+  float ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ss = fmaf(xv[i], xv[i], ss);
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+  const float r = 1.0f / sqrtf(ss / 128.0f + eps);
+  float gate[8];
+  silu_fast(zv, gate);
+  uint32_t o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float y[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) y[e] = round_bf(wv[2 * i + e] * round_bf(xv[2 * i + e] * r)) * gate[2 * i + e];
+    o[i] = pack_bf16(y[0], y[1]);
+  }
+  store16u(out + (size_t)t * ldo + at, make_uint4(o[0], o[1], o[2], o[3]), aligned);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1503,8 +1532,10 @@ int df_gated_rms_norm_rows(const uint16_t* x, int ldx, const uint16_t* z, int ld
       (reinterpret_cast<uintptr_t>(weight) & 3))
     return DF_BAD_ARGUMENT;
   const long units = (long)tokens * heads;
-  hipLaunchKernelGGL(gated_norm_rows_kernel, dim3((units + 3) / 4), dim3(256), 0, stream, x, ldx, z, ldz, weight, eps,
-                     tokens, heads, out, ldo);
+  const int aligned = aligned16(x) && aligned16(z) && aligned16(weight) && aligned16(out) && ldx % 8 == 0 &&
+                      ldz % 8 == 0 && ldo % 8 == 0;
+  hipLaunchKernelGGL(gated_norm_rows_kernel, dim3((units + 15) / 16), dim3(256), 0, stream, x, ldx, z, ldz, weight, eps,
+                     tokens, heads, out, ldo, aligned);
   DF_RETURN_LAUNCH_STATUS();
 }
 

@@ -266,6 +266,22 @@ def test_gated_rms_norm_rows():
     close(got, want, what="gated norm rows")
 
 
+@pytest.mark.parametrize("tokens,heads,shift,pad", [(1, 1, 0, 0), (3, 5, 0, 0), (5, 3, 2, 0), (16, 1, 0, 2), (17, 32, 8, 8)])
+def test_gated_rms_norm_rows_edges(tokens, heads, shift, pad):
+    """Heads that leave a workgroup's last groups empty, and rows that allow only 4-byte accesses."""
+    gen = torch.Generator().manual_seed(tokens + heads)
+    x, z = (torch.randn((tokens, heads * 128), generator=gen).to(torch.bfloat16) for _ in range(2))
+    w = (1.0 + 0.02 * torch.randn(128, generator=gen)).to(torch.bfloat16)
+
+    def wide(t):
+        v = torch.zeros((tokens, t.shape[1] + shift + pad), dtype=t.dtype, device=DEV)[:, shift:shift + t.shape[1]]
+        return v.copy_(t)
+
+    got = gated_rms_norm_rows(wide(x), wide(z), w.to(DEV), 1e-6, out=wide(torch.zeros_like(x)))
+    want = gated_rms_norm(x.reshape(-1, 128), z.reshape(-1, 128), w, 1e-6).reshape(tokens, -1)
+    close(got, want, what="gated norm rows", flip_frac=1e-3)
+
+
 def _attention_expression(q, k, v, gate, pos0, scale, swish):
     """The reference's rounding in fp32: bf16 scores, bf16 softmax, bf16 output, bf16 gate."""
     p, hq, _ = q.shape
