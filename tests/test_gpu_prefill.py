@@ -282,6 +282,42 @@ def test_gated_rms_norm_rows_edges(tokens, heads, shift, pad):
     close(got, want, what="gated norm rows", flip_frac=1e-3)
 
 
+@pytest.mark.parametrize("tokens,hq,hkv,half,pos0,shift", [
+    (1, 4, 1, 4, 0, 0), (3, 4, 1, 8, 5, 4), (7, 8, 2, 16, 30000, 0), (9, 4, 1, 32, 11, 0), (5, 12, 3, 128, 2, 4),
+    (2047, 4, 1, 32, 0, 0), (2049, 4, 1, 32, 3, 0)])
+def test_qk_norm_rope_prefill_edges(tokens, hq, hkv, half, pos0, shift):
+    """Rotations from 8 dims to the whole head, tokens on both sides of the workgroup's change
+    from one to four with a remainder, and rows that allow only 8-byte accesses."""
+    from deltaforge_amd.prefill import qk_norm_rope_prefill
+    print(f"qk edges {tokens} {hq} {hkv} {half} {pos0} {shift}", flush=True)
+    gen = torch.Generator().manual_seed(tokens + half)
+    kc, vc = hq * 512, hq * 512 + hkv * 256
+    proj = torch.randn((tokens, vc + hkv * 256), generator=gen).to(torch.bfloat16)
+    qn, kn = ((0.1 * torch.randn(256, generator=gen)).to(torch.bfloat16) for _ in range(2))
+    inv = 10000.0 ** (-torch.arange(half) / half)
+    wide = torch.zeros((tokens, proj.shape[1] + shift), dtype=torch.bfloat16, device=DEV)[:, shift:].copy_(proj)
+    k_cache, v_cache = (torch.zeros((hkv, pos0 + tokens + 1, 256), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    q = qk_norm_rope_prefill(wide, qn.to(DEV), kn.to(DEV), inv.to(DEV), k_cache, v_cache, num_q_heads=hq, k_col=kc,
+                             v_col=vc, pos0=pos0)
+    bf = lambda t: t.to(torch.bfloat16).float()
+    ang = (pos0 + torch.arange(tokens, dtype=torch.float32)).unsqueeze(1) * inv
+    c, s = (bf(f(torch.cat([ang, ang], -1))).unsqueeze(1) for f in (torch.cos, torch.sin))
+
+    def want(x, w):
+        x = x.float()
+        n = bf(x * torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-6).float() * (1 + w.float()))
+        r = n[..., :2 * half]
+        rotated = torch.cat([-r[..., half:], r[..., :half]], -1)
+        return torch.cat([bf(bf(r * c) + bf(rotated * s)), n[..., 2 * half:]], -1)
+
+    close(q, want(proj[:, :kc].reshape(tokens, hq, 512)[..., :256], qn), what="queries", flip_frac=1e-3)
+    k = want(proj[:, kc:vc].reshape(tokens, hkv, 256), kn).transpose(0, 1)
+    close(k_cache[:, pos0:-1], k, what="keys", flip_frac=1e-3)
+    assert torch.equal(v_cache[:, pos0:-1].cpu(), proj[:, vc:].reshape(tokens, hkv, 256).transpose(0, 1)), "values"
+    for cache in (k_cache, v_cache):
+        assert not cache[:, :pos0].any() and not cache[:, -1].any(), "other rows"
+
+
 def _attention_expression(q, k, v, gate, pos0, scale, swish):
     """The reference's rounding in fp32: bf16 scores, bf16 softmax, bf16 output, bf16 gate."""
     p, hq, _ = q.shape
