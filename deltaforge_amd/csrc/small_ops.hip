@@ -1,6 +1,7 @@
 // Elementwise / row ops of the slot surface and the decode-loop glue, for gfx950.
 #include "common.h"
 #include "deltaforge_hip.h"
+#include "int4_block.h"
 
 namespace df {
 
@@ -32,6 +33,88 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const uint16_t* __restric
     const float scaled = v * r;
     out[row * n + k] = f2bf(scaled * (1.0f + bf2f(w[k])));
   }
+}
+
+// The same with a wave to a row and the row in registers, V chunks of 512 elements: one pass, 16-byte
+// accesses, no barrier. Rows of 2560 with the residual: 1 row 4.2 us (a workgroup to a row,
+// 2-byte accesses, two passes) -> 3.2, 717 rows 6.1 -> 4.6, 4096 rows 20.3 -> 13.0 (84 MB), 16384 rows
+// 106 -> 60.
+template <bool ADD, int V>
+__global__ __launch_bounds__(256) void rms_norm_wave_kernel(const uint16_t* __restrict__ x,
+                                                            const uint16_t* __restrict__ residual,
+                                                            const uint16_t* __restrict__ w, float eps, int rows, int n,
+                                                            uint16_t* __restrict__ resid_out,
+                                                            uint16_t* __restrict__ out) {
+  const int row = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+  if (row >= rows) return;
+  const int k0 = (threadIdx.x & 63) * 8;
+  const size_t base = (size_t)row * n + k0;
+  uint4 xv[V], rv[V], wv[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    xv[i] = make_uint4(0, 0, 0, 0);
+    rv[i] = wv[i] = xv[i];
+    if (k0 + i * 512 < n) {
+      xv[i] = *reinterpret_cast<const uint4*>(x + base + i * 512);
+      if constexpr (ADD) rv[i] = *reinterpret_cast<const uint4*>(residual + base + i * 512);
+      wv[i] = *reinterpret_cast<const uint4*>(w + k0 + i * 512);
+    }
+  }
+  float ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    uint32_t v[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+    const uint32_t r[4] = {rv[i].x, rv[i].y, rv[i].z, rv[i].w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float a = __uint_as_float(v[j] << 16), b = __uint_as_float(v[j] & 0xFFFF0000u);
+      if constexpr (ADD) {
+        v[j] = pack_bf16(a + __uint_as_float(r[j] << 16), b + __uint_as_float(r[j] & 0xFFFF0000u));
+        a = __uint_as_float(v[j] << 16), b = __uint_as_float(v[j] & 0xFFFF0000u);
+      }
+      ss = fmaf(a, a, ss);
+      ss = fmaf(b, b, ss);
+    }
+    if constexpr (ADD) {
+      xv[i] = make_uint4(v[0], v[1], v[2], v[3]);
+      if (k0 + i * 512 < n) *reinterpret_cast<uint4*>(resid_out + base + i * 512) = xv[i];
+    }
+  }
+  const float scale = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(n) + eps);
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const uint32_t v[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w}, g[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
+    uint32_t o[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      o[j] = pack_bf16(__uint_as_float(v[j] << 16) * scale * (1.0f + __uint_as_float(g[j] << 16)),
+                   __uint_as_float(v[j] & 0xFFFF0000u) * scale * (1.0f + __uint_as_float(g[j] & 0xFFFF0000u)));
+    if (k0 + i * 512 < n) *reinterpret_cast<uint4*>(out + base + i * 512) = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
+constexpr int kRmsWaveMax = 8 * 512;  // the longest row that a wave holds
+
+// Both by rows and alignment: see the kernels.
+template <bool ADD>
+void launch_rms_norm(const uint16_t* x, const uint16_t* residual, const uint16_t* w, float eps, int rows, int n,
+                     uint16_t* resid_out, uint16_t* out, hipStream_t stream) {
+  const uintptr_t all = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
+                        reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual) |
+                        reinterpret_cast<uintptr_t>(resid_out);
+  if (n % 8 || n > kRmsWaveMax || (all & 15)) {
+    hipLaunchKernelGGL(rms_norm_kernel<ADD>, dim3(rows), dim3(256), 0, stream, x, residual, w, eps, n, resid_out, out);
+    return;
+  }
+  using Kernel = decltype(&rms_norm_wave_kernel<ADD, 1>);
+  constexpr Kernel kernels[8] = {rms_norm_wave_kernel<ADD, 1>, rms_norm_wave_kernel<ADD, 2>,
+                                 rms_norm_wave_kernel<ADD, 3>, rms_norm_wave_kernel<ADD, 4>,
+                                 rms_norm_wave_kernel<ADD, 5>, rms_norm_wave_kernel<ADD, 6>,
+                                 rms_norm_wave_kernel<ADD, 7>, rms_norm_wave_kernel<ADD, 8>};
+  // fewer rows than 4 waves on each CU: one wave to a workgroup spreads them over the chip
+  const int waves = rows > 1024 ? 4 : 1;
+  hipLaunchKernelGGL(kernels[(n - 1) / 512], dim3((rows + waves - 1) / waves), dim3(waves * 64), 0, stream, x, residual,
+                     w, eps, rows, n, resid_out, out);
 }
 
 __global__ void silu_mul_kernel(const uint16_t* __restrict__ gate, const uint16_t* __restrict__ up, size_t n,
@@ -232,15 +315,14 @@ extern "C" {
 
 int df_rms_norm(const uint16_t* x, const uint16_t* w, float eps, int rows, int n, uint16_t* out, hipStream_t stream) {
   if (!x || !w || !out || rows < 1 || n < 1) return DF_BAD_ARGUMENT;
-  hipLaunchKernelGGL(rms_norm_kernel<false>, dim3(rows), dim3(256), 0, stream, x, nullptr, w, eps, n, nullptr, out);
+  launch_rms_norm<false>(x, nullptr, w, eps, rows, n, nullptr, out, stream);
   DF_RETURN_LAUNCH_STATUS();
 }
 
 int df_add_rms_norm(const uint16_t* x, const uint16_t* residual, const uint16_t* w, float eps, int rows, int n,
                     uint16_t* resid_out, uint16_t* out, hipStream_t stream) {
   if (!x || !residual || !w || !resid_out || !out || rows < 1 || n < 1) return DF_BAD_ARGUMENT;
-  hipLaunchKernelGGL(rms_norm_kernel<true>, dim3(rows), dim3(256), 0, stream, x, residual, w, eps, n, resid_out,
-                     out);
+  launch_rms_norm<true>(x, residual, w, eps, rows, n, resid_out, out, stream);
   DF_RETURN_LAUNCH_STATUS();
 }
 

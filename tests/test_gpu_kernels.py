@@ -46,6 +46,25 @@ def repack(w: synth.CanonicalInt4) -> ops.Int4Weight:
     return ops.int4_repack(w.packed.to(DEV), w.scale.to(DEV))
 
 
+@pytest.mark.parametrize("rows,n,shift", [
+    (1, 8, 0), (3, 504, 0), (5, 520, 0), (1025, 1032, 0), (7, 2560, 0), (2, 4096, 0), (2, 4104, 0), (3, 30, 0),
+    (3, 2560, 4)])
+def test_rms_norm_edges(rows, n, shift):
+    """Rows a wave holds (remainders of its 512-element chunks, its longest, a last workgroup
+    that is not full) and rows it does not: too long, not a multiple of 8, not 16-byte aligned."""
+    gen = torch.Generator().manual_seed(rows + n)
+    rand = lambda *s: torch.randn(s, generator=gen).to(torch.bfloat16)
+    x, r, w = rand(rows, n), rand(rows, n), rand(n) * 0.1
+
+    def dev(t):
+        return torch.zeros(t.numel() + shift, dtype=t.dtype, device=DEV)[shift:].copy_(t.flatten()).view(t.shape)
+
+    close(ops.rms_norm(dev(x), dev(w), 1e-6), rms_norm(x, w, 1e-6), what="norm", flip_frac=1e-2)
+    resid, got = ops.add_rms_norm(dev(x), dev(r), dev(w), 1e-6)
+    assert torch.equal(resid.cpu(), x + r), "sum"
+    close(got, rms_norm(x + r, w, 1e-6), what="sum's norm", flip_frac=1e-2)
+
+
 # -- int4 ---------------------------------------------------------------------------------
 
 
