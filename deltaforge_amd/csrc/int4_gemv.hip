@@ -12,7 +12,7 @@
 //
 // Work split: a workgroup of 8 waves owns NT 16-column tiles; the 8/NT waves that share a
 // tile split its K range, and their fp32 partials are summed in LDS in a fixed order. Each
-// wave keeps 12 groups (8 for the logits epilogue) in flight, 1 KB of weights each. Each group
+// wave keeps up to 10 groups in flight, 1 KB of weights each. Each group
 // is one fully coalesced 1 KB load (64 lanes x 16 B).
 //
 // Arithmetic is the reference's (kernels/visible_int4_head.py:187-199): every weight is
@@ -34,15 +34,16 @@ namespace df {
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
 constexpr int kMaxRows = 16;
-// Groups in flight per wave. 12 puts a whole K range of the decode's MLP shapes (9 to 10
-// groups per wave at 1 row, 9 to 20 at 16) in flight at once or nearly: MLP block 23.5 ->
-// 22.3 us at 1 row and 35.4 -> 33.8 us at 16 rows, against 8. The head's 20-group ranges ran
-// 1.6 to 2.7 % slower with 12 than with 8 (and 16 or 20 were slower everywhere), so the logits
-// epilogue keeps 8.
-template <int EPI>
-constexpr int depth_of() { return EPI == DF_EPI_LOGITS ? 8 : 12; }
+// Groups in flight per wave, or half as many where a wave has no more: the decode's shapes have 4 to
+// 10 groups a wave at 1 row and 9 to 20 at 16, so a range is one or two full sets with few repeats.
+// Against 12 for all but the head's 8: down 9216 x 2560 6.6 -> 6.3 us at 1 row, head 71.2 -> 68.6, a
+// 4096 x 2560 product (4 groups a wave) 6.1 -> 5.6.
+constexpr int kDepth = 10;
 constexpr int kNormChunks = 3;  // RMSNorm prologue: K <= kNormChunks * kThreads * 8 = 12288
 constexpr int kRowChunks = 5;   // ... one wave per row when K <= kRowChunks * 64 * 8 = 2560
+// A prologue's forms: one chunk of a row to a thread, several (norms of K > 4096), a wave to a row (more
+// than 4 rows)
+constexpr int kShortRow = 0, kLongRow = 1, kManyRows = 2;
 constexpr int kGemvLds = 100 * 1024;  // LDS bytes a workgroup may take
 
 struct GemvSmem {
@@ -67,8 +68,106 @@ __host__ __device__ inline GemvSmem gemv_smem(int rows, int kx, int nt) {
 // Prologues: this workgroup's K range of the bf16 activation rows, into LDS.
 // ---------------------------------------------------------------------------------------
 
-template <int PRO, bool WROWS>
-DF_DEVICE void gemv_prologue(const DfInt4GemvArgs& p, uint16_t* xs, int xs_ld, float* red, int k0, int kc) {
+// A prologue's operands go into registers before the weight loads are issued: loads return in
+// order, so a norm whose row was asked for after the weights would wait for all of them, and the
+// sum, its barrier and the scaling (with the norm weight's own round trip after the sum) came on top
+// of the stream instead of under it. What does not fit here is loaded in pro_finish.
+// 1 row, weights in cache where they fit: in_proj 2560 x 12352 8.5 -> 6.9 us, gate|up 2560 x 18432
+// 11.3 -> 10.5, head 2560 x 248320 74.3 -> 68.6; 16 rows: in_proj 13.0 -> 11.2, gate|up 15.0 -> 14.0; 8 rows
+// of the head 117 -> 95 (with kDepth's change). The plain copy keeps its loads behind the weights':
+// before them they delay the stream and have no sum to hide (down, 4 rows, 7.6 -> 8.1 us).
+template <int PRO, int EPI, int FORM>
+struct Pro {
+  static constexpr bool WROWS = FORM == kManyRows;
+  static constexpr bool kNorm = PRO == DF_PRO_RMSNORM || PRO == DF_PRO_ADD_RMSNORM;
+  static constexpr bool kTwo = PRO == DF_PRO_ADD_RMSNORM || PRO == DF_PRO_GATED_RMSNORM;
+  // 16-byte chunks of the rows a thread takes early: the plain copy's and the gated norm's of all
+  // rows, the norms' of one row (a wave's row with WROWS)
+  static constexpr int kX = kNorm ? (WROWS ? kRowChunks : FORM == kShortRow ? 1 : kNormChunks) : WROWS ? 4 : 1;
+  static constexpr int kEarly = kNorm && !WROWS ? 1 : kX;  // (4096 elements; longer rows' other chunks later)
+  static constexpr int kRows = kNorm && WROWS && EPI != DF_EPI_LOGITS ? 2 : 1;  // rows a wave takes early
+  uint4 x[kRows][kX], r[kTwo ? kRows : 1][kTwo ? kX : 1], w[PRO == DF_PRO_NONE ? 1 : kX];
+};
+
+template <int PRO, int EPI, int FORM>
+DF_DEVICE void pro_issue(const DfInt4GemvArgs& p, Pro<PRO, EPI, FORM>& o, int k0, int kc) {
+  using P = Pro<PRO, EPI, FORM>;
+  constexpr bool WROWS = P::WROWS;
+  const int tid = threadIdx.x;
+  if constexpr (PRO == DF_PRO_NONE) return;
+  if constexpr (P::kNorm) {
+    const int first = WROWS ? tid & 63 : tid, step = WROWS ? 64 : kThreads, nchunks = p.K / 8;
+#pragma unroll
+    for (int i = 0; i < P::kRows; ++i) {
+      const int m = WROWS ? (tid >> 6) + i * kWaves : 0;
+#pragma unroll
+      for (int j = 0; j < P::kEarly; ++j) {
+        const int c = first + j * step;
+        o.x[i][j] = make_uint4(0u, 0u, 0u, 0u);
+        if constexpr (P::kTwo) o.r[i][j] = make_uint4(0u, 0u, 0u, 0u);
+        if (c < nchunks && m < p.rows) {
+          o.x[i][j] = load16(p.x + (size_t)m * p.ldx + c * 8);
+          if constexpr (P::kTwo) o.r[i][j] = load16(p.x2 + (size_t)m * p.ldx2 + c * 8);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < P::kEarly; ++j) {
+      const int k = (first + j * step) * 8;
+      o.w[j] = make_uint4(0u, 0u, 0u, 0u);
+      if (k >= k0 && k < k0 + kc) o.w[j] = load16(p.norm_w + k);
+    }
+  } else {
+    const int per = kc / 8;
+#pragma unroll
+    for (int j = 0; j < P::kX; ++j) {
+      const int u = tid + j * kThreads;
+      if (u < p.rows * per) {
+        const int m = u / per, k = k0 + (u - m * per) * 8;
+        o.x[0][j] = load16(p.x + (size_t)m * p.ldx + k);
+        o.r[0][j] = load16(p.x2 + (size_t)m * p.ldx2 + k);
+        o.w[j] = load16(p.norm_w + (k % kGroup));
+      }
+    }
+  }
+}
+
+// bf16(x + residual) of 8 elements (reference.py:735 feeding the next norm)
+DF_DEVICE uint4 add8(const uint4& x, const uint4& r) {
+  const uint32_t a[4] = {x.x, x.y, x.z, x.w}, b[4] = {r.x, r.y, r.z, r.w};
+  uint32_t o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    o[i] = pack_bf16(__uint_as_float(a[i] << 16) + __uint_as_float(b[i] << 16),
+                     __uint_as_float(a[i] & 0xFFFF0000u) + __uint_as_float(b[i] & 0xFFFF0000u));
+  return make_uint4(o[0], o[1], o[2], o[3]);
+}
+DF_DEVICE float sum_squares(const uint4& x, float ss) {
+  const uint32_t a[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float lo = __uint_as_float(a[i] << 16), hi = __uint_as_float(a[i] & 0xFFFF0000u);
+    ss += lo * lo;
+    ss += hi * hi;
+  }
+  return ss;
+}
+// bf16((x r) (1 + w)) (reference.py:92-96)
+DF_DEVICE uint4 scale8(const uint4& x, const uint4& w, float r) {
+  const uint32_t a[4] = {x.x, x.y, x.z, x.w}, b[4] = {w.x, w.y, w.z, w.w};
+  uint32_t o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    o[i] = pack_bf16(__uint_as_float(a[i] << 16) * r * (1.0f + __uint_as_float(b[i] << 16)),
+                     __uint_as_float(a[i] & 0xFFFF0000u) * r * (1.0f + __uint_as_float(b[i] & 0xFFFF0000u)));
+  return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+template <int PRO, int EPI, int FORM>
+DF_DEVICE void pro_finish(const DfInt4GemvArgs& p, Pro<PRO, EPI, FORM>& o, uint16_t* xs, int xs_ld, float* red, int k0,
+                          int kc) {
+  using P = Pro<PRO, EPI, FORM>;
+  constexpr bool WROWS = P::WROWS;
   const int tid = threadIdx.x;
   if (p.rows < kMaxRows) {
     for (int kk = tid * 8; kk < kc; kk += kThreads * 8)
@@ -80,176 +179,96 @@ DF_DEVICE void gemv_prologue(const DfInt4GemvArgs& p, uint16_t* xs, int xs_ld, f
       for (int kk = tid * 8; kk < kc; kk += kThreads * 8)
         *reinterpret_cast<uint4*>(xs + m * xs_ld + kk) = load16(src + kk);
     }
-  } else if constexpr (PRO == DF_PRO_RMSNORM || PRO == DF_PRO_ADD_RMSNORM) {
-    // RMSNorm with the (1 + w) scale over the whole row (reference.py:92-96); with ADD the
-    // row is first bf16(x + residual) (reference.py:735 feeding the next norm). Each thread
-    // owns up to kNormChunks 8-element chunks of the row, loaded once (16-byte loads) and
-    // kept in registers between the sum of squares and the scaling.
-    const bool write_h =
-        (PRO == DF_PRO_ADD_RMSNORM) && p.h_out && blockIdx.x == 0 && blockIdx.y == 0;
-    const int nchunks = p.K / 8;
-    if (WROWS && nchunks <= 64 * kRowChunks) {
-      // Many rows (the WROWS instance): one wave per row (rows w, w + 8, ...), the row and the
-      // norm weight of this workgroup's K range loaded at once into the wave's registers, its
-      // sum of squares reduced within the wave. Rows proceed in parallel with no block-wide
-      // reduction (and no second memory round trip) per row; the sum's order differs from the
-      // block form's only in fp32 rounding. Few rows keep the block form: this one holds more
-      // registers, and the occupancy it costs outweighs what it saves for one row.
-      const int lane = tid & 63, wave = tid >> 6;
-      for (int m = wave; m < p.rows; m += kWaves) {
-        const uint16_t* xr = p.x + (size_t)m * p.ldx;
-        const uint16_t* rr = p.x2 + (size_t)m * p.ldx2;
-        uint32_t v[kRowChunks][4];
-        uint4 wreg[kRowChunks];
-#pragma unroll
-        for (int j = 0; j < kRowChunks; ++j) {
-          const int c = lane + 64 * j, k = c * 8;
-          wreg[j] = make_uint4(0u, 0u, 0u, 0u);
-          v[j][0] = v[j][1] = v[j][2] = v[j][3] = 0u;
-          if (c < nchunks) {
-            const uint4 raw = load16(xr + k);
-            v[j][0] = raw.x, v[j][1] = raw.y, v[j][2] = raw.z, v[j][3] = raw.w;
-            if constexpr (PRO == DF_PRO_ADD_RMSNORM) {
-              const uint4 rraw = load16(rr + k);
-              const uint32_t rw[4] = {rraw.x, rraw.y, rraw.z, rraw.w};
-#pragma unroll
-              for (int e2 = 0; e2 < 4; ++e2) {
-                const uint16_t lo = f2bf(bf2f(static_cast<uint16_t>(v[j][e2])) + bf2f(static_cast<uint16_t>(rw[e2])));
-                const uint16_t hi = f2bf(bf2f(static_cast<uint16_t>(v[j][e2] >> 16)) +
-                                         bf2f(static_cast<uint16_t>(rw[e2] >> 16)));
-                v[j][e2] = lo | (static_cast<uint32_t>(hi) << 16);
-              }
-            }
-            if (k >= k0 && k < k0 + kc) wreg[j] = load16(p.norm_w + k);
-          }
-        }
-        float ss = 0.0f;
-#pragma unroll
-        for (int j = 0; j < kRowChunks; ++j) {
-          const int c = lane + 64 * j;
-          if (c < nchunks) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const float val = bf2f(static_cast<uint16_t>(v[j][e >> 1] >> (16 * (e & 1))));
-              ss += val * val;
-            }
-            if (write_h)
-              *reinterpret_cast<uint4*>(p.h_out + (size_t)m * p.K + c * 8) = make_uint4(v[j][0], v[j][1], v[j][2], v[j][3]);
-          }
-        }
-        ss = wave_sum(ss);
-        const float r = 1.0f / sqrtf(ss / static_cast<float>(p.K) + p.eps);
-#pragma unroll
-        for (int j = 0; j < kRowChunks; ++j) {
-          const int c = lane + 64 * j, k = c * 8;
-          if (c < nchunks && k >= k0 && k < k0 + kc) {
-            const uint32_t ww[4] = {wreg[j].x, wreg[j].y, wreg[j].z, wreg[j].w};
-            uint32_t o[4];
-#pragma unroll
-            for (int e2 = 0; e2 < 4; ++e2) {
-              uint16_t pr[2];
-#pragma unroll
-              for (int h = 0; h < 2; ++h) {
-                const float scaled = bf2f(static_cast<uint16_t>(v[j][e2] >> (16 * h))) * r;
-                pr[h] = f2bf(scaled * (1.0f + bf2f(static_cast<uint16_t>(ww[e2] >> (16 * h)))));
-              }
-              o[e2] = pr[0] | (static_cast<uint32_t>(pr[1]) << 16);
-            }
-            *reinterpret_cast<uint4*>(xs + m * xs_ld + (k - k0)) = make_uint4(o[0], o[1], o[2], o[3]);
-          }
-        }
-      }
-    } else
-    for (int m = 0; m < p.rows; ++m) {
-      const uint16_t* xr = p.x + (size_t)m * p.ldx;
-      const uint16_t* rr = p.x2 + (size_t)m * p.ldx2;
-      uint32_t v[kNormChunks][4];  // the row as packed bf16 (bf16(x + r) is exact in bf16)
+  } else if constexpr (P::kNorm) {
+    // RMSNorm with the (1 + w) scale over the whole row; with ADD the row is first
+    // bf16(x + residual). Few rows: every thread holds chunks of the row and the sum is the
+    // workgroup's. WROWS, many rows: one wave per row (rows w, w + 8, ...), its sum reduced within
+    // the wave, so rows proceed in parallel with no block-wide reduction; it holds more
+    // registers, which costs more than it saves for one row. The two orders of the sum
+    // differ only in fp32 rounding.
+    const bool write_h = (PRO == DF_PRO_ADD_RMSNORM) && p.h_out && blockIdx.x == 0 && blockIdx.y == 0;
+    const int first = WROWS ? tid & 63 : tid, step = WROWS ? 64 : kThreads, nchunks = p.K / 8;
+    auto row = [&](int m, uint4 (&x)[P::kX], const uint4* r) {
       float ss = 0.0f;
 #pragma unroll
-      for (int j = 0; j < kNormChunks; ++j) {
-        const int c = tid + j * kThreads;
-        if (c < nchunks) {
-          const uint4 raw = load16(xr + c * 8);
-          v[j][0] = raw.x, v[j][1] = raw.y, v[j][2] = raw.z, v[j][3] = raw.w;
-          if constexpr (PRO == DF_PRO_ADD_RMSNORM) {
-            const uint4 rraw = load16(rr + c * 8);
-            const uint32_t rw[4] = {rraw.x, rraw.y, rraw.z, rraw.w};
-#pragma unroll
-            for (int e2 = 0; e2 < 4; ++e2) {
-              const uint16_t lo = f2bf(bf2f(static_cast<uint16_t>(v[j][e2])) + bf2f(static_cast<uint16_t>(rw[e2])));
-              const uint16_t hi = f2bf(bf2f(static_cast<uint16_t>(v[j][e2] >> 16)) +
-                                       bf2f(static_cast<uint16_t>(rw[e2] >> 16)));
-              v[j][e2] = lo | (static_cast<uint32_t>(hi) << 16);
-            }
-          }
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float val = bf2f(static_cast<uint16_t>(v[j][e >> 1] >> (16 * (e & 1))));
-            ss += val * val;
-          }
-          if (write_h)
-            *reinterpret_cast<uint4*>(p.h_out + (size_t)m * p.K + c * 8) = make_uint4(v[j][0], v[j][1], v[j][2], v[j][3]);
-        }
+      for (int j = 0; j < P::kX; ++j) {
+        const int c = first + j * step;
+        if constexpr (P::kTwo) x[j] = add8(x[j], r[j]);
+        ss = sum_squares(x[j], ss);  // absent chunks are zero
+        if (write_h && c < nchunks) *reinterpret_cast<uint4*>(p.h_out + (size_t)m * p.K + c * 8) = x[j];
       }
-      ss = block_sum<kWaves>(ss, red);
-      const float r = 1.0f / sqrtf(ss / static_cast<float>(p.K) + p.eps);
+      ss = WROWS ? wave_sum(ss) : block_sum<kWaves>(ss, red);
+      const float rs = 1.0f / sqrtf(ss / static_cast<float>(p.K) + p.eps);
 #pragma unroll
-      for (int j = 0; j < kNormChunks; ++j) {
-        const int c = tid + j * kThreads;
-        const int k = c * 8;
-        if (c < nchunks && k >= k0 && k < k0 + kc) {
-          const uint4 wraw = load16(p.norm_w + k);
-          const uint32_t ww[4] = {wraw.x, wraw.y, wraw.z, wraw.w};
-          uint32_t o[4];
+      for (int j = 0; j < P::kX; ++j) {
+        const int k = (first + j * step) * 8;
+        if (k >= k0 && k < k0 + kc) *reinterpret_cast<uint4*>(xs + m * xs_ld + (k - k0)) = scale8(x[j], o.w[j], rs);
+      }
+    };
+    if constexpr (P::kEarly < P::kX) {
 #pragma unroll
-          for (int e2 = 0; e2 < 4; ++e2) {
-            uint16_t pr[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const float scaled = bf2f(static_cast<uint16_t>(v[j][e2] >> (16 * h))) * r;
-              pr[h] = f2bf(scaled * (1.0f + bf2f(static_cast<uint16_t>(ww[e2] >> (16 * h)))));
-            }
-            o[e2] = pr[0] | (static_cast<uint32_t>(pr[1]) << 16);
-          }
-          *reinterpret_cast<uint4*>(xs + m * xs_ld + (k - k0)) = make_uint4(o[0], o[1], o[2], o[3]);
+      for (int j = P::kEarly; j < P::kX; ++j) {
+        const int c = first + j * step, k = c * 8;
+        o.x[0][j] = o.w[j] = make_uint4(0u, 0u, 0u, 0u);
+        if constexpr (P::kTwo) o.r[0][j] = o.x[0][j];
+        if (c < nchunks) {
+          o.x[0][j] = load16(p.x + k);
+          if constexpr (P::kTwo) o.r[0][j] = load16(p.x2 + k);
         }
+        if (k >= k0 && k < k0 + kc) o.w[j] = load16(p.norm_w + k);
       }
     }
-  } else {  // DF_PRO_GATED_RMSNORM: one 128-group == one value head (reference.py:115-121)
-    // 8 elements per thread; a head is 16 consecutive lanes, reduced with lane shuffles.
-    for (int m = 0; m < p.rows; ++m) {
-      for (int c = tid; c < kc / 8; c += kThreads) {
-        const int k = k0 + c * 8;
-        const uint4 xraw = load16(p.x + (size_t)m * p.ldx + k);
-        const uint4 zraw = load16(p.x2 + (size_t)m * p.ldx2 + k);
-        const uint4 wraw = load16(p.norm_w + (k % kGroup));
-        const uint32_t xw[4] = {xraw.x, xraw.y, xraw.z, xraw.w};
-        const uint32_t zw[4] = {zraw.x, zraw.y, zraw.z, zraw.w};
-        const uint32_t ww[4] = {wraw.x, wraw.y, wraw.z, wraw.w};
-        float v[8];
-        float ss = 0.0f;
+    int m = WROWS ? tid >> 6 : 0;
+    const int next = WROWS ? kWaves : 1;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          v[e] = bf2f(static_cast<uint16_t>(xw[e >> 1] >> (16 * (e & 1))));
-          ss += v[e] * v[e];
+    for (int i = 0; i < P::kRows; ++i, m += next)
+      if (m < p.rows) row(m, o.x[i], P::kTwo ? o.r[i] : nullptr);
+    for (; m < p.rows; m += next) {
+      uint4 x[P::kX], r[P::kX];
+#pragma unroll
+      for (int j = 0; j < P::kX; ++j) {
+        const int c = first + j * step;
+        x[j] = r[j] = make_uint4(0u, 0u, 0u, 0u);
+        if (c < nchunks) {
+          x[j] = load16(p.x + (size_t)m * p.ldx + c * 8);
+          if constexpr (P::kTwo) r[j] = load16(p.x2 + (size_t)m * p.ldx2 + c * 8);
         }
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) ss += __shfl_xor(ss, off, 64);
-        const float r = 1.0f / sqrtf(ss / 128.0f + p.eps);
-        uint32_t o[4];
-#pragma unroll
-        for (int e2 = 0; e2 < 4; ++e2) {
-          uint16_t pr[2];
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const int e = e2 * 2 + h;
-            const float t = round_bf(bf2f(static_cast<uint16_t>(ww[e2] >> (16 * h))) * round_bf(v[e] * r));
-            pr[h] = f2bf(t * silu(bf2f(static_cast<uint16_t>(zw[e2] >> (16 * h)))));
-          }
-          o[e2] = pr[0] | (static_cast<uint32_t>(pr[1]) << 16);
-        }
-        *reinterpret_cast<uint4*>(xs + m * xs_ld + c * 8) = make_uint4(o[0], o[1], o[2], o[3]);
       }
+      row(m, x, r);
+    }
+  } else {
+    const int per = kc / 8, total = p.rows * per;
+    auto put = [&](int u, const uint4& x, const uint4& z, const uint4& w) {
+      const int m = u / per, c = u - m * per;
+      // one 128-group is one value head (reference.py:115-121): 16 consecutive lanes, 8 elements each
+      float ss = sum_squares(x, 0.0f);
+#pragma unroll
+      for (int off = 1; off < 16; off <<= 1) ss += __shfl_xor(ss, off, 64);
+      const float r = 1.0f / sqrtf(ss / 128.0f + p.eps);
+      const uint32_t xw[4] = {x.x, x.y, x.z, x.w}, zw[4] = {z.x, z.y, z.z, z.w}, ww[4] = {w.x, w.y, w.z, w.w};
+      uint32_t out[4];
+#pragma unroll
+      for (int e2 = 0; e2 < 4; ++e2) {
+        float g[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const float xe = bf2f(static_cast<uint16_t>(xw[e2] >> (16 * h)));
+          const float t = round_bf(bf2f(static_cast<uint16_t>(ww[e2] >> (16 * h))) * round_bf(xe * r));
+          g[h] = t * silu(bf2f(static_cast<uint16_t>(zw[e2] >> (16 * h))));
+        }
+        out[e2] = pack_bf16(g[0], g[1]);
+      }
+      *reinterpret_cast<uint4*>(xs + m * xs_ld + c * 8) = make_uint4(out[0], out[1], out[2], out[3]);
+    };
+#pragma unroll
+    for (int j = 0; j < P::kX; ++j) {
+      const int u = tid + j * kThreads;
+      if (u < total) put(u, o.x[0][j], o.r[0][j], o.w[j]);
+    }
+    for (int u = tid + P::kX * kThreads; u < total; u += kThreads) {
+      const int m = u / per, k = k0 + (u - m * per) * 8;
+      put(u, load16(p.x + (size_t)m * p.ldx + k), load16(p.x2 + (size_t)m * p.ldx2 + k),
+          load16(p.norm_w + (k % kGroup)));
     }
   }
   __syncthreads();
@@ -281,11 +300,11 @@ DF_DEVICE void gemv_epilogue(const DfInt4GemvArgs& p, const float* y, int col0, 
   }
 }
 
-template <int PRO, int EPI, int NT, bool WROWS>
-__global__ __launch_bounds__(kThreads) void w4_gemv_kernel(DfInt4GemvArgs p) {
+template <int PRO, int EPI, int NT, int FORM, int DEPTH>
+__global__ __launch_bounds__(kThreads, FORM == kManyRows || PRO == DF_PRO_NONE ? 2 : 4)
+void w4_gemv_kernel(DfInt4GemvArgs p) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int KS = kWaves / NT;
-  constexpr int kDepth = depth_of<EPI>();
   constexpr int COLS = NT * kTileCols;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int tsub = wave % NT, kpart = wave / NT;
@@ -303,23 +322,23 @@ __global__ __launch_bounds__(kThreads) void w4_gemv_kernel(DfInt4GemvArgs p) {
   const unsigned char* wp = p.w + ((size_t)tile * G + gx0) * kBlockBytes + lane * 16;
   const uint16_t* sp = p.s + ((size_t)tile * G + gx0) * kTileCols + (lane & 15);
 
-  // Weights do not depend on the activations: put the first groups in flight before the
-  // prologue so HBM is busy while the norm is computed. Refills are clamped to the last
-  // group of the range (a repeat read of a cached block) so the pipeline is branch-free.
-  const bool has_work = g_lo < g_hi;
-  const int g_last = g_hi - 1;
-  uint4 wb[kDepth];
-  uint16_t sb[kDepth];
-  if (has_work) {
+  // The prologue's operands, then the first groups of weights, all in flight at once; the
+  // prologue then waits for its own loads only (no branch around the weights', which would make
+  // the wait one for everything). Refills are clamped to the last group of the range (a
+  // repeat read of a cached block) so the pipeline is branch-free; a wave without groups reads one.
+  Pro<PRO, EPI, FORM> pro;
+  pro_issue<PRO, EPI, FORM>(p, pro, gx0 * kGroup, ngx * kGroup);
+  const int g_last = max(g_hi - 1, 0);
+  uint4 wb[DEPTH];
+  uint16_t sb[DEPTH];
 #pragma unroll
-    for (int u = 0; u < kDepth; ++u) {
-      const int g = min(g_lo + u, g_last);
-      wb[u] = load16(wp + (size_t)g * kBlockBytes);
-      sb[u] = sp[g * kTileCols];
-    }
+  for (int u = 0; u < DEPTH; ++u) {
+    const int g = min(g_lo + u, g_last);
+    wb[u] = load16(wp + (size_t)g * kBlockBytes);
+    sb[u] = sp[g * kTileCols];
   }
 
-  gemv_prologue<PRO, WROWS>(p, xs, L.xs_ld, red, gx0 * kGroup, ngx * kGroup);
+  pro_finish<PRO, EPI, FORM>(p, pro, xs, L.xs_ld, red, gx0 * kGroup, ngx * kGroup);
 
   const int col = lane & 15;   // A row, B/C column, scale column
   const int slot = lane >> 4;  // K slot of A and B; C row block
@@ -340,12 +359,12 @@ __global__ __launch_bounds__(kThreads) void w4_gemv_kernel(DfInt4GemvArgs p) {
   };
 
   int g0 = g_lo;
-  for (; g0 + kDepth <= g_hi; g0 += kDepth) {
+  for (; g0 + DEPTH < g_hi; g0 += DEPTH) {
 #pragma unroll
-    for (int u = 0; u < kDepth; ++u) {
+    for (int u = 0; u < DEPTH; ++u) {
       const uint4 wv = wb[u];
       const uint16_t sv = sb[u];
-      const int gn = min(g0 + u + kDepth, g_last);
+      const int gn = min(g0 + u + DEPTH, g_last);
       wb[u] = load16(wp + (size_t)gn * kBlockBytes);
       sb[u] = sp[gn * kTileCols];
       group_mac(wv, sv, g0 + u);
@@ -353,7 +372,7 @@ __global__ __launch_bounds__(kThreads) void w4_gemv_kernel(DfInt4GemvArgs p) {
   }
   // Tail: the remaining groups are already in wb[0 .. g_hi - g0).
 #pragma unroll
-  for (int u = 0; u < kDepth; ++u) {
+  for (int u = 0; u < DEPTH; ++u) {
     if (g0 + u < g_hi) group_mac(wb[u], sb[u], g0 + u);
   }
 
@@ -463,10 +482,16 @@ static hipError_t launch_gemv(const DfInt4GemvArgs& a, hipStream_t stream) {
   const GemvSmem L = gemv_smem(a.rows, min(gps, G) * kGroup, NT);
   dim3 grid(a.N / (NT * kTileCols), a.ksplit);
   constexpr bool kNorm = PRO == DF_PRO_RMSNORM || PRO == DF_PRO_ADD_RMSNORM;
-  if (kNorm && a.rows > 4 && a.K <= kRowChunks * 64 * 8)
-    hipLaunchKernelGGL((w4_gemv_kernel<PRO, EPI, NT, kNorm>), grid, dim3(kThreads), L.total, stream, a);
+  const int per = (min(gps, G) + kWaves / NT - 1) / (kWaves / NT);  // groups a wave
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), L.total, stream, a); };
+  if (PRO != DF_PRO_NONE && a.rows > 4 && (!kNorm || a.K <= kRowChunks * 64 * 8))
+    go(w4_gemv_kernel<PRO, EPI, NT, kManyRows, kDepth>);
+  else if (kNorm && a.K > kThreads * 8)
+    go(w4_gemv_kernel<PRO, EPI, NT, kLongRow, kDepth>);
+  else if (per <= kDepth / 2)
+    go(w4_gemv_kernel<PRO, EPI, NT, kShortRow, kDepth / 2>);
   else
-    hipLaunchKernelGGL((w4_gemv_kernel<PRO, EPI, NT, false>), grid, dim3(kThreads), L.total, stream, a);
+    go(w4_gemv_kernel<PRO, EPI, NT, kShortRow, kDepth>);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.ksplit == 1) return e;
   hipLaunchKernelGGL((w4_reduce_kernel<EPI>), dim3(a.N / 64), dim3(256), 0, stream, a);

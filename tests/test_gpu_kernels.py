@@ -16,7 +16,7 @@ from deltaforge_amd import ops, synth
 from deltaforge_amd.config import qwen3_5_4b_config
 from oracle import ops as oracle_ops
 from oracle.int4 import dequant_gemv, dequantise_int4_k_major_np
-from oracle.model import apply_partial_rope, causal_conv, rms_norm
+from oracle.model import apply_partial_rope, causal_conv, gated_rms_norm, rms_norm
 
 pytestmark = pytest.mark.gpu
 
@@ -123,6 +123,46 @@ def test_int4_gemv_k_split_reuses_its_workspace(epilogue):
     again = ops.int4_gemv(x0.to(DEV), weight, epilogue=epilogue, plan=plans[0], ws=ws,
                           res=res0.to(DEV) if epilogue == N.EPI_RESIDUAL else None)
     assert torch.equal(again, got0)
+
+
+@pytest.mark.parametrize("prologue,epilogue,rows,k,nt", [
+    (N.PRO_NONE, N.EPI_STORE, 1, 256, 1), (N.PRO_NONE, N.EPI_STORE, 6, 1280, 8), (N.PRO_NONE, N.EPI_STORE, 16, 1536, 8),
+    (N.PRO_RMSNORM, N.EPI_STORE, 1, 256, 1), (N.PRO_RMSNORM, N.EPI_STORE, 3, 4096, 4),
+    (N.PRO_RMSNORM, N.EPI_STORE, 2, 4352, 2), (N.PRO_RMSNORM, N.EPI_STORE, 9, 512, 8),
+    (N.PRO_RMSNORM, N.EPI_LOGITS, 16, 2560, 8), (N.PRO_ADD_RMSNORM, N.EPI_LOGITS, 5, 2816, 8),
+    (N.PRO_ADD_RMSNORM, N.EPI_STORE, 1, 4352, 1), (N.PRO_ADD_RMSNORM, N.EPI_STORE, 4, 2560, 4),
+    (N.PRO_ADD_RMSNORM, N.EPI_STORE, 16, 2304, 2), (N.PRO_ADD_RMSNORM, N.EPI_STORE, 5, 4352, 8),
+    (N.PRO_GATED_RMSNORM, N.EPI_STORE, 1, 256, 1), (N.PRO_GATED_RMSNORM, N.EPI_STORE, 3, 4096, 8),
+    (N.PRO_GATED_RMSNORM, N.EPI_STORE, 7, 512, 4), (N.PRO_GATED_RMSNORM, N.EPI_STORE, 16, 2304, 2)])
+def test_int4_gemv_prologue_forms(prologue, epilogue, rows, k, nt):
+    """Rows and widths on both sides of what a prologue loads ahead of the weights, and from no
+    group to several sets of groups in a wave. The norm's bf16 results may round the other way where
+    the fp32 sum's order does (one in thousands, 2^-8 each), so the product is held normwise, like the
+    MLP block."""
+    print(f"gemv prologue {prologue} {rows} {k} {nt}", flush=True)
+    gen = torch.Generator().manual_seed(rows + k)
+    rand = lambda *s: torch.randn(s, generator=gen).to(torch.bfloat16)
+    w = synth.draw_int4(gen, k, 128)
+    x, x2 = rand(rows, k), rand(rows, k)
+    nw = rand(128 if prologue == N.PRO_GATED_RMSNORM else k) * 0.1
+    h_out = torch.zeros((rows, k), dtype=torch.bfloat16, device=DEV)
+    kw = {} if prologue == N.PRO_NONE else {"norm_w": nw.to(DEV)}
+    if prologue in (N.PRO_ADD_RMSNORM, N.PRO_GATED_RMSNORM):
+        kw["x2"] = x2.to(DEV)
+    if prologue == N.PRO_ADD_RMSNORM:
+        kw["h_out"] = h_out
+    got = ops.int4_gemv(x.to(DEV), repack(w), prologue=prologue, epilogue=epilogue,
+                        plan=ops.GemvPlan(nt, 1, k // 128, 0), **kw)
+    if prologue == N.PRO_RMSNORM:
+        x = rms_norm(x, nw, 1e-6)
+    elif prologue == N.PRO_ADD_RMSNORM:
+        assert torch.equal(h_out.cpu(), x + x2)
+        x = rms_norm(x + x2, nw, 1e-6)
+    elif prologue == N.PRO_GATED_RMSNORM:
+        x = gated_rms_norm(x.reshape(-1, 128), x2.reshape(-1, 128), nw, 1e-6).reshape(rows, k)
+    want = dequant_gemv(x, w.packed, w.scale, 128).float()
+    err = float((got.float().cpu() - want).abs().max())
+    assert err <= ATOL + RTOL * float(want.abs().max()), f"max abs err {err:.4g}"
 
 
 def test_int4_gemv_is_deterministic_across_runs():
