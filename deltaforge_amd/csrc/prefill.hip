@@ -6,10 +6,12 @@
 // - the chunked gated delta rule;
 // - GatedRMSNorm over rows;
 // - q/k RMSNorm + partial RoPE over rows, which also writes the KV cache;
-// - causal GQA attention with the reference's bf16 softmax rounding.
+// - causal GQA attention in one pass over the keys.
 //
 // Every rounding point is the reference's forward over a sequence (reference.py:496-550,
-// 610-677, 692-735). Only fp32 summation order differs.
+// 610-677, 692-735), but one: from the 33rd position on, attention rounds exp(s - m) to bf16 and
+// divides by the sum after the product, where the reference rounds the quotient (the same relative
+// rounding). Otherwise only fp32 summation order differs.
 #include <math.h>
 
 #include "common.h"

@@ -10,7 +10,7 @@ the HIP kernels of ``csrc/prefill.hip``:
 - the chunked delta rule (64-token chunks, exact in real arithmetic to the scan);
 - GatedRMSNorm over rows;
 - q/k norm + RoPE, which also writes the KV cache;
-- causal GQA attention with the reference's bf16 softmax rounding.
+- causal GQA attention, one pass over the keys.
 
 Then RMSNorm, the tied head and the argmax of the last position.
 
