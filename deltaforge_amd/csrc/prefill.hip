@@ -12,6 +12,7 @@
 // 610-677, 692-735), but one: from the 33rd position on, attention rounds exp(s - m) to bf16 and
 // divides by the sum after the product, where the reference rounds the quotient (the same relative
 // rounding). Otherwise only fp32 summation order differs.
+#include <float.h>
 #include <math.h>
 
 #include "common.h"
@@ -1208,6 +1209,7 @@ __global__ __launch_bounds__(kAtThreads, 1) void attn_prefill_kernel(DfAttnPrefi
   const int pos_lo = p.pos0 + t0, pos_hi = pos_lo + 31;  // the wave's positions
   const bool pow2 = flags & kAtPow2Scale;
   const float cexp = pow2 ? p.scale * kLog2e : kLog2e;
+  const float masked = p.scale < 0.0f ? INFINITY : -INFINITY;  // a score that the scale makes -inf
 
   f32x16 o[8];
 #pragma unroll
@@ -1236,7 +1238,7 @@ __global__ __launch_bounds__(kAtThreads, 1) void attn_prefill_kernel(DfAttnPrefi
     if (key0 + 31 > pos_lo) {
 #pragma unroll
       for (int e = 0; e < 16; ++e)
-        s[e] = key0 + (e & 3) + 8 * (e >> 2) + 4 * half <= pos ? s[e] : -INFINITY;
+        s[e] = key0 + (e & 3) + 8 * (e >> 2) + 4 * half <= pos ? s[e] : masked;
     }
   };
   auto prob = [&](float r, float mc) { return __builtin_amdgcn_exp2f(fmaf(r, cexp, -mc)); };
@@ -1588,8 +1590,12 @@ int df_attention_prefill(const DfAttnPrefillArgs* a, hipStream_t stream) {
   if (!aligned16(a->q) || !aligned16(a->k_cache) || !aligned16(a->v_cache) || a->ld_out < a->num_q_heads * kHd ||
       a->gate_kind < 0 || a->gate_kind > 1)
     return DF_BAD_ARGUMENT;
+  DfAttnPrefillArgs args = *a;
+  // A scale of zero would turn a masked score into NaN. The smallest normal number leaves every
+  // exp(s - m) of scores below 1e29 at 1, as zero does.
+  if (args.scale == 0.0f) args.scale = FLT_MIN;
   int e = 0;
-  const bool pow2 = a->scale > 0.0f && frexpf(a->scale, &e) == 0.5f;
+  const bool pow2 = args.scale > 0.0f && frexpf(args.scale, &e) == 0.5f;
   auto mult = [](const void* ptr, int ld, int align) {
     return (reinterpret_cast<uintptr_t>(ptr) % align) == 0 && ld % (align / 2) == 0;
   };
@@ -1597,7 +1603,7 @@ int df_attention_prefill(const DfAttnPrefillArgs* a, hipStream_t stream) {
                     (mult(a->gate, a->ld_gate, 8) && a->gate_head_stride % 4 == 0 ? kAtVecGate : 0) |
                     (mult(a->out, a->ld_out, 8) ? kAtVecOut : 0);
   hipLaunchKernelGGL(attn_prefill_kernel, dim3((a->tokens + 31) / 32 * a->num_kv_heads), dim3(kAtThreads), kAtLds,
-                     stream, *a, flags);
+                     stream, args, flags);
   DF_RETURN_LAUNCH_STATUS();
 }
 

@@ -334,11 +334,13 @@ def _attention_expression(q, k, v, gate, pos0, scale, swish):
 
 
 # row blocks of 32 positions, key blocks of 64 in two sets of 32, the first 32 positions, later
-# chunks; a scale that is no power of two; gate and output rows that allow no 8-byte access
+# chunks; a scale that is no power of two, zero or negative (a masked key stays masked); gate and output
+# rows that allow no 8-byte access
 @pytest.mark.parametrize("tokens,pos0,scale,swish,shift", [
     (1, 0, 1 / 16, False, 0), (31, 0, 1 / 16, True, 0), (33, 0, 0.07, False, 0), (64, 0, 1 / 16, False, 1),
     (97, 0, 0.05, True, 3), (1, 31, 1 / 16, False, 0), (2, 31, 1 / 16, False, 0), (40, 30, 1 / 16, False, 0),
-    (1, 64, 1 / 16, False, 0), (70, 200, 1 / 16, False, 2), (130, 63, 0.3, False, 0)])
+    (1, 64, 1 / 16, False, 0), (70, 200, 1 / 16, False, 2), (130, 63, 0.3, False, 0), (97, 0, -0.05, False, 0),
+    (40, 30, 0.0, False, 0), (130, 63, -1 / 16, True, 2)])
 def test_attention_prefill_edges(tokens, pos0, scale, swish, shift):
     print(f"attention prefill {tokens} at {pos0}", flush=True)
     from deltaforge_amd import prefill as P
