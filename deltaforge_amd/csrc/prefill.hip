@@ -15,6 +15,8 @@
 #include <float.h>
 #include <math.h>
 
+#include <algorithm>
+
 #include "common.h"
 #include "deltaforge_hip.h"
 #include "int4_block.h"
@@ -976,6 +978,17 @@ __global__ __launch_bounds__(kScanThreads) void delta_scan_kernel(DfDeltaPrefill
   for (int r = 0; r < 4; ++r) gstate[(size_t)(16 * wave + 4 * q4 + r) * kDk + col0 + n16] = S[r];
 }
 
+// The outputs from the scratch to `out`, for an `out` over `mixed`'s memory, which every workgroup of the
+// scan reads to the end: [tokens][width], 4 channels a thread.
+__global__ __launch_bounds__(256) void delta_out_kernel(const uint16_t* __restrict__ from, int tokens, int width,
+                                                        uint16_t* __restrict__ out, int ldo) {
+  const int per = width / 4, t = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= per) return;
+  for (int row = t; row < tokens; row += gridDim.y)
+    *reinterpret_cast<uint2*>(out + (size_t)row * ldo + c * 4) =
+        *reinterpret_cast<const uint2*>(from + (size_t)row * width + c * 4);
+}
+
 // ---------------------------------------------------------------------------------------
 // GatedRMSNorm over rows (reference.py:115-121)
 // ---------------------------------------------------------------------------------------
@@ -1525,7 +1538,17 @@ int df_causal_conv_prefill(const uint16_t* x, int ldx, int tokens, int channels,
 size_t df_delta_rule_prefill_workspace_bytes(int tokens, int num_v_heads) {
   if (tokens < 1 || num_v_heads < 1) return 0;
   const size_t chunks = (size_t)(tokens + kCk - 1) / kCk;
-  return chunks * num_v_heads * kPrepFloats * sizeof(float);
+  return chunks * num_v_heads * (kPrepFloats * sizeof(float) + kCk * kDk * sizeof(uint16_t));
+}
+
+// Whether two sets of `rows` rows (lda and ldb elements apart, wa and wb long) share memory. Rows of one
+// stride whose columns lie beside each other do not.
+static bool rows_overlap(const uint16_t* a, int lda, int wa, const uint16_t* b, int ldb, int wb, int rows) {
+  const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
+  if (a0 + ((size_t)(rows - 1) * lda + wa) * 2 <= b0 || b0 + ((size_t)(rows - 1) * ldb + wb) * 2 <= a0) return false;
+  if (lda != ldb) return true;
+  const size_t ld = (size_t)lda * 2, apart = b0 >= a0 ? (b0 - a0) % ld : (ld - (a0 - b0) % ld) % ld;
+  return apart < (size_t)wa * 2 || apart + (size_t)wb * 2 > ld;
 }
 
 int df_delta_rule_prefill(const DfDeltaPrefillArgs* a, void* workspace, size_t workspace_bytes, hipStream_t stream) {
@@ -1544,8 +1567,18 @@ int df_delta_rule_prefill(const DfDeltaPrefillArgs* a, void* workspace, size_t w
   float* scratch = reinterpret_cast<float*>(workspace);
   const int aligned = aligned16(a->mixed) && a->ld_mixed % 8 == 0;  // rows allow 16-byte loads
   hipLaunchKernelGGL(delta_prep_kernel, dim3(chunks, a->num_v_heads), dim3(256), 0, stream, *a, scratch, aligned);
-  hipLaunchKernelGGL(delta_scan_kernel, dim3(a->num_v_heads, kDk / kScanVs), dim3(kScanThreads), 0, stream, *a,
+  const int width = a->num_v_heads * kDk;
+  DfDeltaPrefillArgs scan = *a;
+  const bool staged = rows_overlap(a->mixed, a->ld_mixed, channels, a->out, a->ld_out, width, a->tokens);
+  if (staged) {
+    scan.out = reinterpret_cast<uint16_t*>(scratch + (size_t)chunks * a->num_v_heads * kPrepFloats);
+    scan.ld_out = width;
+  }
+  hipLaunchKernelGGL(delta_scan_kernel, dim3(a->num_v_heads, kDk / kScanVs), dim3(kScanThreads), 0, stream, scan,
                      static_cast<const float*>(scratch), aligned);
+  if (staged)
+    hipLaunchKernelGGL(delta_out_kernel, dim3((width / 4 + 255) / 256, std::min(a->tokens, 65535)), dim3(256), 0, stream,
+                       scan.out, a->tokens, width, a->out, a->ld_out);
   DF_RETURN_LAUNCH_STATUS();
 }
 

@@ -101,7 +101,7 @@ def delta_rule_prefill(mixed: Tensor, a: Tensor, b: Tensor, A_log: Tensor, dt_bi
                        num_k_heads: int, out: Tensor | None = None) -> Tensor:
     """Chunked gated delta rule over ``mixed`` ``[P, q|k|v]`` (the conv output); ``a``, ``b``
     ``[P, >= Hv]`` raw gate projections (strided rows, one stride); ``state`` ``[Hv, 128, 128]``
-    fp32 updated in place. Returns the core output ``[P, Hv * 128]`` bf16."""
+    fp32 updated in place. Returns the core output ``[P, Hv * 128]`` bf16; ``out`` may lie over ``mixed``."""
     if state.dim() != 3 or state.dtype != torch.float32 or not state.is_contiguous() or state.shape[1:] != (128, 128):
         raise ValueError(f"state must be a contiguous fp32 [Hv, 128, 128], got {state.dtype} {tuple(state.shape)}")
     hv = state.shape[0]
@@ -118,8 +118,6 @@ def delta_rule_prefill(mixed: Tensor, a: Tensor, b: Tensor, A_log: Tensor, dt_bi
     ops._check_dtype(op, "dt_bias", dt_bias, BF16, hv)
     if out is None:
         out = torch.empty((tokens, hv * 128), dtype=BF16, device=mixed.device)
-    elif out.untyped_storage().data_ptr() == mixed.untyped_storage().data_ptr():
-        mixed = mixed.clone()  # the scan reads q, k and v while it writes out
     ops.require_gpus(op, mixed, a, b, A_log, dt_bias, state, out)
     nbytes = int(N.lib().df_delta_rule_prefill_workspace_bytes(tokens, hv))
     ws = ops.workspace(mixed.device, nbytes, "delta_prefill")

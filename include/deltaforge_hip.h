@@ -289,7 +289,7 @@ int df_causal_conv_prefill(const uint16_t* x, int ldx, int tokens, int channels,
  * head h on key head h / (Hv / Hk), beta = bf16(sigmoid(b)), g = -exp(A_log) softplus(a +
  * dt_bias). mixed: the conv output [tokens][ld_mixed] = q | k | v channels; a, b: the raw
  * bf16 gate projections [tokens][ld_ab]; state [Hv][128][128] fp32 read and updated;
- * out [tokens][ld_out] bf16 (head h at column 128 h). */
+ * out [tokens][ld_out] bf16 (head h at column 128 h); it may lie over `mixed`. */
 typedef struct DfDeltaPrefillArgs {
   const uint16_t* mixed;
   const uint16_t* a;
@@ -301,8 +301,10 @@ typedef struct DfDeltaPrefillArgs {
   int ld_mixed, ld_ab, ld_out;
   int tokens, num_k_heads, num_v_heads;
 } DfDeltaPrefillArgs;
-/* Workspace (bytes) for `tokens` tokens and Hv value heads: per (64-token chunk, head), the
- * five 64 x 128 fp32 state-independent products of the chunk and its total decay. */
+/* Workspace (bytes) for `tokens` tokens and Hv value heads: per (64-token chunk, head), the ten
+ * 16 x 16 fp32 blocks of each of the chunk's two lower triangles (T and QK), four fp32 factors a token
+ * and the total decay, and room for the chunk's 64 x 128 bf16 outputs, which wait there when `out`
+ * lies over `mixed`. */
 size_t df_delta_rule_prefill_workspace_bytes(int tokens, int num_v_heads);
 int df_delta_rule_prefill(const DfDeltaPrefillArgs* args, void* workspace, size_t workspace_bytes,
                           hipStream_t stream);

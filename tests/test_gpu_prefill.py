@@ -255,6 +255,29 @@ def test_delta_rule_prefill_edges(tokens, hk, hv, shift, pad):
         assert torch.equal(run(0, tokens, st3, out=wide[:, :hv * 128]), got), "out within mixed"
 
 
+@pytest.mark.parametrize("tokens,at,ld", [(1, 0, 0), (65, 1024, 0), (300, 128, 0), (300, 512, 1024), (65, 1536, 0)])
+def test_delta_rule_prefill_out_over_mixed_by_address(tokens, at, ld):
+    """``out`` as a tensor of another storage over ``mixed``'s memory: inside its columns, one row and
+    several, with a stride of its own (``ld``), and beside it in a wider buffer."""
+    hk, hv = 2, 4
+    mixed, ab, A_log, dt_bias, state = _delta_case(tokens, seed=tokens + at, hk=hk, hv=hv)
+    width = mixed.shape[1]
+    buf = torch.zeros((tokens + 1, width + hv * 128), dtype=torch.bfloat16, device=DEV)
+    rows = buf[:tokens, :width]
+    rows.copy_(mixed)
+    args = [t.to(DEV) for t in (ab, A_log, dt_bias)]
+
+    def run(st, **kw):
+        return delta_rule_prefill(rows, args[0][:, :hv], args[0][:, hv:], args[1], args[2], st, num_k_heads=hk, **kw)
+
+    st, st2 = state.to(DEV), state.to(DEV)
+    want = run(st)
+    out = torch.as_strided(buf, (tokens, hv * 128), (ld or buf.stride(0), 1), at)
+    out = torch.from_dlpack(out)
+    assert out.untyped_storage().data_ptr() != buf.untyped_storage().data_ptr() or at == 0
+    assert torch.equal(run(st2, out=out), want) and torch.equal(st2, st)
+
+
 def test_gated_rms_norm_rows():
     gen = torch.Generator().manual_seed(9)
     tokens, heads = 70, 32
