@@ -80,8 +80,13 @@ def _check_dtype(op: str, name: str, t: Tensor, dtype: torch.dtype, numel: int |
 
 
 def _stream(t: Tensor) -> int:
-    """The device's current stream as a handle, without the ``torch.cuda.Stream`` object."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    """The device's current stream as a handle, without the ``torch.cuda.Stream`` object. A tensor
+    that is on no GPU (index -1, for which the raw call answers with the current GPU's stream) is an
+    error: its pointer must not reach a kernel."""
+    index = t.get_device()
+    if index < 0:
+        raise ValueError(f"Expected a cuda device, but got: {t.device}")
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 _WORKSPACES: dict[tuple, Tensor] = {}

@@ -220,6 +220,28 @@ def test_bad_shapes_raise_value_error_before_the_device_check(call):
         call()
 
 
+@pytest.mark.parametrize("call", [
+    lambda ops: ops.int4_dequant(ops.Int4Weight(torch.zeros(2 * 1024, dtype=torch.uint8), torch.zeros(32, dtype=BF16), 256, 16)),
+    lambda ops: ops.silu_mul(torch.zeros(8, dtype=BF16), torch.zeros(8, dtype=BF16)),
+])
+def test_a_host_tensor_has_no_stream(call, monkeypatch):
+    """An op whose own check does not cover the tensor that it takes the stream of (a weight, ``up``)
+    raises at the stream, before any host pointer reaches the library."""
+    from deltaforge_amd import ops
+
+    class Library:
+        def __getattr__(self, name):
+            def reached(*args):
+                raise AssertionError(f"{name} was reached with host pointers")
+            return reached
+
+    monkeypatch.setattr(ops, "require_gpu", lambda t, op: None)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0)
+    monkeypatch.setattr(N, "lib", Library)
+    with pytest.raises((ValueError, RuntimeError)):
+        call(ops)
+
+
 def test_delta_and_attention_ops_validate_before_device():
     c = mid_config(num_layers=4)
     hv, hk, dk = c.linear_num_value_heads, c.linear_num_key_heads, 128
