@@ -115,11 +115,16 @@ DF_DEVICE void dma4(const void* gaddr, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(gaddr), "s"(lds_base)
                : "memory", "m0");
 }
-// y[i] = x / (1 + e^-x) of N values from the hardware's exp2 and a reciprocal with one Newton step
-// instead of expf and an IEEE division: 8 VALU instead of about 40. Far out, where the quotient
-// nears fp32's smallest numbers, it is silu() (one branch for the N: one for each took 10 us of
-// the 717 x 2560 x 18432 SwiGLU product's 82). Of the 65536 bf16 inputs every one gives the same
-// bf16 as silu(). With silu() the SwiGLU epilogue takes 6 us more of a 128 x 256 tile's 40, the conv
+// The same with the global address as a uniform base plus the lane's offset.
+DF_DEVICE void dma16s(const void* base, uint32_t offset, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_base)
+               : "memory", "m0");
+}
+// y[i] = x / (1 + e^-x) of N values where y is rounded to bf16 at once: from the hardware's exp2 and a
+// reciprocal with one Newton step instead of expf and an IEEE division, 8 VALU instead of about 40. Far
+// out, where the quotient nears fp32's smallest numbers, it is silu() (one branch for the N: one for each
+// took 10 us of the 717 x 2560 x 18432 SwiGLU product's 82). Of the 65536 bf16 inputs every one gives the
+// same bf16 as silu(). With silu() the SwiGLU epilogue takes 6 us more of a 128 x 256 tile's 40, the conv
 // 17 more of 25 (4096 tokens, 8192 channels).
 template <int N>
 DF_DEVICE void silu_fast(const float (&x)[N], float (&y)[N]) {
@@ -137,10 +142,29 @@ DF_DEVICE void silu_fast(const float (&x)[N], float (&y)[N]) {
       if (x[i] < -80.0f) y[i] = silu(x[i]);
   }
 }
-// The same with the global address as a uniform base plus the lane's offset.
-DF_DEVICE void dma16s(const void* base, uint32_t offset, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_base)
-               : "memory", "m0");
+// The same where y goes on in fp32, in about 19 VALU: every finite bf16 input gives silu()'s own bits. e^-x
+// is 2^n 2^f with the product -x log2 e in two parts (silu_fast rounds it: up to 3e-6 of the quotient
+// at -80, 3e-7 at -4), and a residual step each corrects the reciprocal and the quotient.
+template <int N>
+DF_DEVICE void silu_bits(const float (&x)[N], float (&y)[N]) {
+#pragma clang fp contract(off)
+  float low = x[0];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float c = fminf(x[i], 104.0f);  // e^-x is nothing beside 1 long before
+    const float t = -1.44269504f * c, n = rintf(t);
+    const float f = (t - n) + fmaf(-1.92596299e-8f, c, fmaf(-1.44269504f, c, -t));
+    const float d = 1.0f + ldexpf(__builtin_amdgcn_exp2f(f), static_cast<int>(n));
+    const float r0 = __builtin_amdgcn_rcpf(d), r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
+    const float q = x[i] * r;
+    y[i] = copysignf(fmaf(fmaf(-d, q, x[i]), r, q), x[i]);  // (-0 stays so)
+    low = fminf(low, x[i]);
+  }
+  if (__builtin_expect(low < -80.0f, 0)) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (x[i] < -80.0f) y[i] = silu(x[i]);
+  }
 }
 template <int N>
 DF_DEVICE void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
@@ -994,7 +1018,8 @@ __global__ __launch_bounds__(256) void delta_out_kernel(const uint16_t* __restri
 // ---------------------------------------------------------------------------------------
 
 // Sixteen lanes to a head, 8 dims each (16-byte accesses where `aligned`, else 4-byte ones), so
-// the sum is four exchanges. 4096 tokens of 32 heads, 101 MB: 38 us (a wave to a head) -> 19.
+// the sum is four exchanges. 4096 tokens of 32 heads, 101 MB: 38 us (a wave to a head) -> 21 (24 with silu()
+// for the gate).
 __global__ __launch_bounds__(256) void gated_norm_rows_kernel(const uint16_t* __restrict__ x, int ldx,
                                                               const uint16_t* __restrict__ z, int ldz,
                                                               const uint16_t* __restrict__ w, float eps, int tokens,
@@ -1015,7 +1040,7 @@ __global__ __launch_bounds__(256) void gated_norm_rows_kernel(const uint16_t* __
   for (int off = 8; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
   const float r = 1.0f / sqrtf(ss / 128.0f + eps);
   float gate[8];
-  silu_fast(zv, gate);
+  silu_bits(zv, gate);
   uint32_t o[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {

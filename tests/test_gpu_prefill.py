@@ -305,6 +305,26 @@ def test_gated_rms_norm_rows_edges(tokens, heads, shift, pad):
     close(got, want, what="gated norm rows", flip_frac=1e-3)
 
 
+def test_gated_rms_norm_rows_gate_is_fp32():
+    """The gate's SiLU goes into the product unrounded, so results are compared with the product in 64
+    bits, rounded once. x is +-1 and eps 0, so that the norm is x itself; a head has one z, all of a
+    weight's mantissas. z is every bf16 from -80 to 104. The gate is off by 3 x 2^-23 at most (2 for e^-z,
+    half for 1 + e^-z, half for the quotient), the product by 2^-24: a result may round the other way only
+    that near to the middle of two bf16."""
+    bits = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    z = bits[(bits.float() >= -80) & (bits.float() <= 104) & (bits.float().abs() > 1e-30)]
+    z = torch.cat([z, z[:-z.numel() % 32]]).reshape(-1, 32, 1).expand(-1, 32, 128).reshape(-1, 32 * 128)
+    x = torch.where(torch.arange(z.shape[1]) % 3 == 0, -1.0, 1.0).to(torch.bfloat16).expand(z.shape).contiguous()
+    w = (1 + torch.arange(128) / 128).to(torch.bfloat16)
+    got = gated_rms_norm_rows(x.to(DEV), z.to(DEV), w.to(DEV), 0.0).cpu()
+    z64 = z.double()
+    want = x.double() * w.double().repeat(32) * (z64 / (1 + torch.exp(-z64)))
+    off = (got.double() - want).abs()
+    spacing = 2.0 ** (torch.floor(torch.log2(want.abs())) - 7)  # of bf16 at want
+    wrong = off > 0.5 * spacing + 3.5 * 2.0**-23 * want.abs()
+    assert not wrong.any(), f"{int(wrong.sum())} results, z from {float(z[wrong].min())} to {float(z[wrong].max())}"
+
+
 @pytest.mark.parametrize("tokens,hq,hkv,half,pos0,shift", [
     (1, 4, 1, 4, 0, 0), (3, 4, 1, 8, 5, 4), (7, 8, 2, 16, 30000, 0), (9, 4, 1, 32, 11, 0), (5, 12, 3, 128, 2, 4),
     (2047, 4, 1, 32, 0, 0), (2049, 4, 1, 32, 3, 0)])
