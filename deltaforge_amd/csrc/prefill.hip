@@ -1090,12 +1090,14 @@ DF_DEVICE void store4(uint16_t* dst, const float x[4]) {
 // One thread group of 32 lanes per (token, slot), 8 dims a lane: slots < Hq are query heads
 // (normed, roped -> q_out), the next Hkv are KV heads (key normed and roped, value copied, both
 // into the cache at pos0 + t). The arithmetic is the decode kernel's norm_rope4 (attention.hip).
-// A workgroup takes `per` tokens with all their slots, so that the angles' cosines and sines, a
-// token's in common, are computed once. 8192 tokens of
-// 16 + 4 heads, 201 MB: 110 us (a wave to a slot, every angle in every head) -> 47; 717 tokens 13 -> 9.6.
-__global__ __launch_bounds__(256) void qk_rows_kernel(DfQkPrefillArgs p, int per, int aligned) {
+// A workgroup takes `per` tokens and `sper` of their slots, whose angles' cosines and sines, a token's in
+// common, are computed once. 8192 tokens of 16 + 4 heads, 201 MB: 103 us (a wave to a slot, every
+// angle in every head) -> 41; 717 tokens 13.1 -> 8.5; 17 tokens 3.9 -> 4.0 (6.9 where a workgroup goes
+// through all 20 slots in three turns).
+__global__ __launch_bounds__(256) void qk_rows_kernel(DfQkPrefillArgs p, int per, int sper, int aligned) {
   __shared__ float2 cs[kQkTokens * kHd / 2];
-  const int l = threadIdx.x & 31, half = p.rotary_dim / 2, slots = p.num_q_heads + p.num_kv_heads;
+  const int l = threadIdx.x & 31, half = p.rotary_dim / 2;
+  const int s0 = blockIdx.y * sper, slots = min(sper, p.num_q_heads + p.num_kv_heads - s0);
   const int t0 = blockIdx.x * per, count = min(per, p.tokens - t0);
   for (int i = threadIdx.x; i < count * half; i += 256) {
     const int t = i / half;
@@ -1110,7 +1112,7 @@ __global__ __launch_bounds__(256) void qk_rows_kernel(DfQkPrefillArgs p, int per
   }
   __syncthreads();
   for (int u = threadIdx.x >> 5; u < count * slots; u += 8) {
-    const int t = u / slots, sl = u - t * slots, g = sl - p.num_q_heads;
+    const int t = u / slots, sl = s0 + u - t * slots, g = sl - p.num_q_heads;
     const bool query = g < 0;
     const uint16_t* row = p.proj + (size_t)(t0 + t) * p.ld_proj + l * 8;
     const size_t cache = ((size_t)(query ? 0 : g) * p.max_len + p.pos0 + t0 + t) * kHd + l * 8;
@@ -1635,9 +1637,14 @@ int df_qk_norm_rope_prefill(const DfQkPrefillArgs* a, hipStream_t stream) {
     return DF_BAD_ARGUMENT;
   const int aligned = aligned16(a->proj) && a->ld_proj % 8 == 0 && a->k_col % 8 == 0 && a->v_col % 8 == 0 &&
                       aligned16(a->q_out) && aligned16(a->k_cache) && aligned16(a->v_cache);
-  // four tokens' angles fill a pass of the workgroup; short prompts need the workgroups
-  const int per = a->tokens >= 2048 ? kQkTokens : 1;
-  hipLaunchKernelGGL(qk_rows_kernel, dim3((a->tokens + per - 1) / per), dim3(256), 0, stream, *a, per, aligned);
+  // Long prompts: four tokens to a workgroup, all their slots. Short ones need the workgroups: one
+  // token and, where they still leave the chip's latency bare, as many slots as a workgroup has thread groups
+  // (20 slots: 512 tokens 7.8 -> 6.7 us, 717 as long, 1500 12.5 -> 13.8 of recomputed angles; 10 slots: 1024
+  // tokens 7.0 -> 6.5).
+  const int slots = a->num_q_heads + a->num_kv_heads, per = a->tokens >= 2048 ? kQkTokens : 1;
+  const int sper = (long)a->tokens * slots <= 12288 ? 8 : slots;
+  hipLaunchKernelGGL(qk_rows_kernel, dim3((a->tokens + per - 1) / per, (slots + sper - 1) / sper), dim3(256), 0, stream, *a,
+                     per, sper, aligned);
   DF_RETURN_LAUNCH_STATUS();
 }
 
