@@ -440,90 +440,60 @@ __global__ __launch_bounds__(128 * WN, 1) void int4_gemm_kernel(DfInt4GemmArgs p
 // order with fp32 sums (the decode step's arithmetic); x(q) is row q - pos0 of the input for
 // q >= pos0, else the history ring (slot q mod 4, zero for positions before the first).
 //
-// A thread walks `per` tokens of V channels with the window in registers, so a row is read
-// 1 + 3 / per times; V = 4 (8-byte loads, four rows in flight) where rows allow it, else 1. The
-// threads of the first tokens also put the last three inputs into the ring, after they have
-// read it. 4096 tokens of 8192 channels, 134 MB, with the ring: 89 + 5 us (a thread to an
-// element, four loads each) -> 30; 717 tokens 14 + 5 -> 9. Walks of 8 and 32 tokens take as long.
-template <int V>
+// A thread walks `per` tokens of a channel, four rows in flight and the window in registers, so a row
+// is read 1 + 3 / per times; the threads of the first tokens also put the last three inputs into the
+// ring, after they have read it. 4096 tokens of 8192 channels, 134 MB, with the ring: 68 us (a thread to an
+// element, four loads each, and a launch for the ring) -> 26; 717 tokens 14.7 -> 7.6; 17 tokens 4.2 -> 2.9. Four
+// channels to a thread in 8-byte accesses are no faster long (27 us) and a longer chain short (17 tokens
+// 5.6).
 __global__ __launch_bounds__(256) void conv_seq_kernel(const uint16_t* __restrict__ x, int ldx, int tokens,
                                                        int channels, const uint16_t* __restrict__ w,
                                                        uint16_t* __restrict__ ring, int pos0,
                                                        uint16_t* __restrict__ out, int ldo, int per) {
 #pragma clang fp contract(off)
-  static_assert(V == 1 || V == 4, "one channel or four");
-  const int c = (blockIdx.x * 256 + threadIdx.x) * V;
+  const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= channels) return;
   const int t0 = blockIdx.y * per, t1 = min(t0 + per, tokens);
-  float wk[V][4];
-#pragma unroll
-  for (int v = 0; v < V; ++v) {
-    const uint2 wt = *reinterpret_cast<const uint2*>(w + (size_t)(c + v) * 4);
-    wk[v][0] = __uint_as_float(wt.x << 16), wk[v][1] = __uint_as_float(wt.x & 0xFFFF0000u);
-    wk[v][2] = __uint_as_float(wt.y << 16), wk[v][3] = __uint_as_float(wt.y & 0xFFFF0000u);
-  }
-  auto load = [&](int t, float (&h)[V]) {
-    const uint16_t* src = x + (size_t)t * ldx + c;
-    if constexpr (V == 4) {
-      const uint2 r = *reinterpret_cast<const uint2*>(src);
-      h[0] = __uint_as_float(r.x << 16), h[1] = __uint_as_float(r.x & 0xFFFF0000u);
-      h[2] = __uint_as_float(r.y << 16), h[3] = __uint_as_float(r.y & 0xFFFF0000u);
-    } else {
-      h[0] = bf2f(*src);
-    }
-  };
-  float h[7][V];  // rows t - 3 .. t + 3
+  const uint2 wt = *reinterpret_cast<const uint2*>(w + (size_t)c * 4);
+  const float wk[4] = {__uint_as_float(wt.x << 16), __uint_as_float(wt.x & 0xFFFF0000u),
+                       __uint_as_float(wt.y << 16), __uint_as_float(wt.y & 0xFFFF0000u)};
+  auto load = [&](int t) { return bf2f(x[(size_t)t * ldx + c]); };
+  float h[7];  // rows t - 3 .. t + 3
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     const int t = t0 - 3 + j;
-    if (t >= 0) {
-      load(t, h[j]);
-    } else {
-#pragma unroll
-      for (int v = 0; v < V; ++v) h[j][v] = bf2f(ring[(size_t)(c + v) * 4 + ((pos0 + t) & 3)]);
-    }
+    h[j] = t >= 0 ? load(t) : bf2f(ring[(size_t)c * 4 + ((pos0 + t) & 3)]);
   }
   for (int t = t0; t < t1; t += 4) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) load(min(t + i, tokens - 1), h[3 + i]);
+    for (int i = 0; i < 4; ++i) h[3 + i] = load(min(t + i, tokens - 1));
+    float s[4], y[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      float s[V], y[V];
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        float acc = h[i][v] * wk[v][0];
-        acc = acc + h[i + 1][v] * wk[v][1];
-        acc = acc + h[i + 2][v] * wk[v][2];
-        acc = acc + h[i + 3][v] * wk[v][3];
-        s[v] = round_bf(acc);
-      }
-      silu_fast(s, y);
-      if (t + i < t1) {
-        uint16_t* dst = out + (size_t)(t + i) * ldo + c;
-        if constexpr (V == 4)
-          *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]));
-        else
-          *dst = f2bf(y[0]);
-      }
+      float acc = h[i] * wk[0];
+      acc = acc + h[i + 1] * wk[1];
+      acc = acc + h[i + 2] * wk[2];
+      acc = acc + h[i + 3] * wk[3];
+      s[i] = round_bf(acc);
     }
+    silu_fast(s, y);
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
+    for (int i = 0; i < 4; ++i)
+      if (t + i < t1) out[(size_t)(t + i) * ldo + c] = f2bf(y[i]);
 #pragma unroll
-      for (int v = 0; v < V; ++v) h[j][v] = h[j + 4][v];
+    for (int j = 0; j < 3; ++j) h[j] = h[j + 4];
   }
   if (t0 == 0) {
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       const int t = tokens - 3 + j;
-      if (t < 0) continue;
-#pragma unroll
-      for (int v = 0; v < V; ++v) ring[(size_t)(c + v) * 4 + ((pos0 + t) & 3)] = x[(size_t)t * ldx + c + v];
+      if (t >= 0) ring[(size_t)c * 4 + ((pos0 + t) & 3)] = x[(size_t)t * ldx + c];
     }
   }
 }
 
 // Tokens a thread walks: long walks read fewer rows twice, short ones fill the chip.
-static int conv_tokens(int tokens) { return tokens >= 2048 ? 16 : 4; }
+static int conv_tokens(int tokens, int channels) { return (long)tokens * channels >= 1 << 23 ? 16 : 4; }
 
 // ---------------------------------------------------------------------------------------
 // chunked gated delta rule (reference.py:403-461 over a sequence)
@@ -1553,12 +1523,9 @@ int df_causal_conv_prefill(const uint16_t* x, int ldx, int tokens, int channels,
   if (!x || !weight || !ring || !out || tokens < 1 || channels < 1 || ldx < channels || ldo < channels || pos0 < 0 ||
       (reinterpret_cast<uintptr_t>(weight) & 7) || tokens > 65535)
     return DF_BAD_ARGUMENT;
-  const bool vec = channels % 4 == 0 && ldx % 4 == 0 && ldo % 4 == 0 && !(reinterpret_cast<uintptr_t>(x) & 7) &&
-                   !(reinterpret_cast<uintptr_t>(out) & 7);
-  const int per = conv_tokens(tokens);
-  const dim3 grid((channels + (vec ? 1023 : 255)) / (vec ? 1024 : 256), (tokens + per - 1) / per);
-  hipLaunchKernelGGL(vec ? conv_seq_kernel<4> : conv_seq_kernel<1>, grid, dim3(256), 0, stream, x, ldx, tokens, channels,
-                     weight, ring, pos0, out, ldo, per);
+  const int per = conv_tokens(tokens, channels);
+  hipLaunchKernelGGL(conv_seq_kernel, dim3((channels + 255) / 256, (tokens + per - 1) / per), dim3(256), 0, stream, x, ldx,
+                     tokens, channels, weight, ring, pos0, out, ldo, per);
   DF_RETURN_LAUNCH_STATUS();
 }
 
