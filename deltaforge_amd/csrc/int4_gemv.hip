@@ -81,8 +81,8 @@ struct Pro {
   static constexpr bool WROWS = FORM == kManyRows;
   static constexpr bool kNorm = PRO == DF_PRO_RMSNORM || PRO == DF_PRO_ADD_RMSNORM;
   static constexpr bool kTwo = PRO == DF_PRO_ADD_RMSNORM || PRO == DF_PRO_GATED_RMSNORM;
-  // 16-byte chunks of the rows a thread takes early: the plain copy's and the gated norm's of all
-  // rows, the norms' of one row (a wave's row with WROWS)
+  // 16-byte chunks of the rows a thread takes early: the gated norm's of all rows, the norms' of one
+  // row (a wave's row with WROWS); the plain copy takes none
   static constexpr int kX = kNorm ? (WROWS ? kRowChunks : FORM == kShortRow ? 1 : kNormChunks) : WROWS ? 4 : 1;
   static constexpr int kEarly = kNorm && !WROWS ? 1 : kX;  // (4096 elements; longer rows' other chunks later)
   static constexpr int kRows = kNorm && WROWS && EPI != DF_EPI_LOGITS ? 2 : 1;  // rows a wave takes early
@@ -484,14 +484,14 @@ static hipError_t launch_gemv(const DfInt4GemvArgs& a, hipStream_t stream) {
   constexpr bool kNorm = PRO == DF_PRO_RMSNORM || PRO == DF_PRO_ADD_RMSNORM;
   const int per = (min(gps, G) + kWaves / NT - 1) / (kWaves / NT);  // groups a wave
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), L.total, stream, a); };
-  if (PRO != DF_PRO_NONE && a.rows > 4 && (!kNorm || a.K <= kRowChunks * 64 * 8))
-    go(w4_gemv_kernel<PRO, EPI, NT, kManyRows, kDepth>);
-  else if (kNorm && a.K > kThreads * 8)
-    go(w4_gemv_kernel<PRO, EPI, NT, kLongRow, kDepth>);
-  else if (per <= kDepth / 2)
-    go(w4_gemv_kernel<PRO, EPI, NT, kShortRow, kDepth / 2>);
-  else
+  [&] {
+    if constexpr (PRO != DF_PRO_NONE)
+      if (a.rows > 4 && (!kNorm || a.K <= kRowChunks * 64 * 8)) return go(w4_gemv_kernel<PRO, EPI, NT, kManyRows, kDepth>);
+    if constexpr (kNorm)
+      if (a.K > kThreads * 8) return go(w4_gemv_kernel<PRO, EPI, NT, kLongRow, kDepth>);
+    if (per <= kDepth / 2) return go(w4_gemv_kernel<PRO, EPI, NT, kShortRow, kDepth / 2>);
     go(w4_gemv_kernel<PRO, EPI, NT, kShortRow, kDepth>);
+  }();
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.ksplit == 1) return e;
   hipLaunchKernelGGL((w4_reduce_kernel<EPI>), dim3(a.N / 64), dim3(256), 0, stream, a);

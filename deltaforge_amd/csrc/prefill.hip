@@ -545,7 +545,6 @@ DF_DEVICE df_f32x4 mfma16(const float4& a, const float4& b, df_f32x4 acc) {
   acc = mfma4(a.z, b.z, acc);
   return mfma4(a.w, b.w, acc);
 }
-DF_DEVICE float4 as_f4(const uint4& v) { return __builtin_bit_cast(float4, v); }
 // 16 bytes from an address that may be only 4-byte aligned.
 DF_DEVICE uint4 load16u(const uint16_t* p, bool aligned) {
   if (aligned) return *reinterpret_cast<const uint4*>(p);
