@@ -34,16 +34,19 @@ namespace df {
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
 constexpr int kMaxRows = 16;
-// Groups in flight per wave, or half as many where a wave has no more: the decode's shapes have 4 to
-// 10 groups a wave at 1 row and 9 to 20 at 16, so a range is one or two full sets with few repeats.
-// Against 12 for all but the head's 8: down 9216 x 2560 6.6 -> 6.3 us at 1 row, head 71.2 -> 68.6, a
-// 4096 x 2560 product (4 groups a wave) 6.1 -> 5.6.
+// Groups in flight per wave (kLongRow: kLongDepth), or half as many where a wave has no more: the
+// decode's shapes have 4 to 10 groups a wave at 1 row and 9 to 20 at 16, so a range is one or two full
+// sets with few repeats. Against 12 for all but the head's 8: down 9216 x 2560 6.6 -> 6.3 us at 1 row,
+// head 71.2 -> 68.6, a 4096 x 2560 product (4 groups a wave) 6.1 -> 5.6.
 constexpr int kDepth = 10;
 constexpr int kNormChunks = 3;  // RMSNorm prologue: K <= kNormChunks * kThreads * 8 = 12288
 constexpr int kRowChunks = 5;   // ... one wave per row when K <= kRowChunks * 64 * 8 = 2560
 // A prologue's forms: one chunk of a row to a thread, several (norms of K > 4096), a wave to a row (more
 // than 4 rows)
 constexpr int kShortRow = 0, kLongRow = 1, kManyRows = 2;
+// kLongRow's chunks leave registers for 8 groups at its two workgroups a CU (10 spill, and cost 4 % at
+// 16 rows of 4352 and 5120).
+constexpr int kLongDepth = 8;
 constexpr int kGemvLds = 100 * 1024;  // LDS bytes a workgroup may take
 
 struct GemvSmem {
@@ -488,7 +491,7 @@ static hipError_t launch_gemv(const DfInt4GemvArgs& a, hipStream_t stream) {
     if constexpr (PRO != DF_PRO_NONE)
       if (a.rows > 4 && (!kNorm || a.K <= kRowChunks * 64 * 8)) return go(w4_gemv_kernel<PRO, EPI, NT, kManyRows, kDepth>);
     if constexpr (kNorm)
-      if (a.K > kThreads * 8) return go(w4_gemv_kernel<PRO, EPI, NT, kLongRow, kDepth>);
+      if (a.K > kThreads * 8) return go(w4_gemv_kernel<PRO, EPI, NT, kLongRow, kLongDepth>);
     if (per <= kDepth / 2) return go(w4_gemv_kernel<PRO, EPI, NT, kShortRow, kDepth / 2>);
     go(w4_gemv_kernel<PRO, EPI, NT, kShortRow, kDepth>);
   }();
