@@ -41,9 +41,10 @@ constexpr int kMaxRows = 16;
 constexpr int kDepth = 10;
 constexpr int kNormChunks = 3;  // RMSNorm prologue: K <= kNormChunks * kThreads * 8 = 12288
 constexpr int kRowChunks = 5;   // ... one wave per row when K <= kRowChunks * 64 * 8 = 2560
+constexpr int kFewChunks = 2;   // ... K <= 1024
 // A prologue's forms: one chunk of a row to a thread, several (norms of K > 4096), a wave to a row (more
-// than 4 rows)
-constexpr int kShortRow = 0, kLongRow = 1, kManyRows = 2;
+// than 4 rows), the same for norms of K <= 1024
+constexpr int kShortRow = 0, kLongRow = 1, kManyRows = 2, kManyShort = 3;
 // kLongRow's chunks leave registers for 8 groups at its two workgroups a CU (10 spill, and cost 4 % at
 // 16 rows of 4352 and 5120).
 constexpr int kLongDepth = 8;
@@ -81,12 +82,13 @@ __host__ __device__ inline GemvSmem gemv_smem(int rows, int kx, int nt) {
 // before them they delay the stream and have no sum to hide (down, 4 rows, 7.6 -> 8.1 us).
 template <int PRO, int EPI, int FORM>
 struct Pro {
-  static constexpr bool WROWS = FORM == kManyRows;
+  static constexpr bool WROWS = FORM >= kManyRows;
   static constexpr bool kNorm = PRO == DF_PRO_RMSNORM || PRO == DF_PRO_ADD_RMSNORM;
   static constexpr bool kTwo = PRO == DF_PRO_ADD_RMSNORM || PRO == DF_PRO_GATED_RMSNORM;
   // 16-byte chunks of the rows a thread takes early: the gated norm's of all rows, the norms' of one
   // row (a wave's row with WROWS); the plain copy takes none
-  static constexpr int kX = kNorm ? (WROWS ? kRowChunks : FORM == kShortRow ? 1 : kNormChunks) : WROWS ? 4 : 1;
+  static constexpr int kNormX[4] = {1, kNormChunks, kRowChunks, kFewChunks};
+  static constexpr int kX = kNorm ? kNormX[FORM] : WROWS ? 4 : 1;
   static constexpr int kEarly = kNorm && !WROWS ? 1 : kX;  // (4096 elements; longer rows' other chunks later)
   static constexpr int kRows = kNorm && WROWS && EPI != DF_EPI_LOGITS ? 2 : 1;  // rows a wave takes early
   uint4 x[kRows][kX], r[kTwo ? kRows : 1][kTwo ? kX : 1], w[PRO == DF_PRO_NONE ? 1 : kX];
@@ -304,7 +306,7 @@ DF_DEVICE void gemv_epilogue(const DfInt4GemvArgs& p, const float* y, int col0, 
 }
 
 template <int PRO, int EPI, int NT, int FORM, int DEPTH>
-__global__ __launch_bounds__(kThreads, FORM == kManyRows || PRO == DF_PRO_NONE ? 2 : 4)
+__global__ __launch_bounds__(kThreads, FORM >= kManyRows || PRO == DF_PRO_NONE ? 2 : 4)
 void w4_gemv_kernel(DfInt4GemvArgs p) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int KS = kWaves / NT;
@@ -488,6 +490,8 @@ static hipError_t launch_gemv(const DfInt4GemvArgs& a, hipStream_t stream) {
   const int per = (min(gps, G) + kWaves / NT - 1) / (kWaves / NT);  // groups a wave
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), L.total, stream, a); };
   [&] {
+    if constexpr (kNorm)
+      if (a.rows > 4 && a.K <= kFewChunks * 64 * 8) return go(w4_gemv_kernel<PRO, EPI, NT, kManyShort, kDepth>);
     if constexpr (PRO != DF_PRO_NONE)
       if (a.rows > 4 && (!kNorm || a.K <= kRowChunks * 64 * 8)) return go(w4_gemv_kernel<PRO, EPI, NT, kManyRows, kDepth>);
     if constexpr (kNorm)

@@ -132,6 +132,8 @@ def test_int4_gemv_k_split_reuses_its_workspace(epilogue):
     (N.PRO_RMSNORM, N.EPI_LOGITS, 16, 2560, 8), (N.PRO_ADD_RMSNORM, N.EPI_LOGITS, 5, 2816, 8),
     (N.PRO_ADD_RMSNORM, N.EPI_STORE, 1, 4352, 1), (N.PRO_ADD_RMSNORM, N.EPI_STORE, 4, 2560, 4),
     (N.PRO_ADD_RMSNORM, N.EPI_STORE, 16, 2304, 2), (N.PRO_ADD_RMSNORM, N.EPI_STORE, 5, 4352, 8),
+    (N.PRO_ADD_RMSNORM, N.EPI_STORE, 5, 256, 1), (N.PRO_ADD_RMSNORM, N.EPI_LOGITS, 16, 1024, 4),
+    (N.PRO_RMSNORM, N.EPI_STORE, 9, 768, 2), (N.PRO_RMSNORM, N.EPI_STORE, 6, 1280, 2),
     (N.PRO_GATED_RMSNORM, N.EPI_STORE, 1, 256, 1), (N.PRO_GATED_RMSNORM, N.EPI_STORE, 3, 4096, 8),
     (N.PRO_GATED_RMSNORM, N.EPI_STORE, 7, 512, 4), (N.PRO_GATED_RMSNORM, N.EPI_STORE, 16, 2304, 2)])
 def test_int4_gemv_prologue_forms(prologue, epilogue, rows, k, nt):
