@@ -440,60 +440,88 @@ __global__ __launch_bounds__(128 * WN, 1) void int4_gemm_kernel(DfInt4GemmArgs p
 // order with fp32 sums (the decode step's arithmetic); x(q) is row q - pos0 of the input for
 // q >= pos0, else the history ring (slot q mod 4, zero for positions before the first).
 //
-// A thread walks `per` tokens of a channel, four rows in flight and the window in registers, so a row
+// A thread walks `per` tokens of V channels, four rows in flight and the window in registers, so a row
 // is read 1 + 3 / per times; the threads of the first tokens also put the last three inputs into the
-// ring, after they have read it. 4096 tokens of 8192 channels, 134 MB, with the ring: 68 us (a thread to an
-// element, four loads each, and a launch for the ring) -> 26; 717 tokens 14.7 -> 7.6; 17 tokens 4.2 -> 2.9. Four
-// channels to a thread in 8-byte accesses are no faster long (27 us) and a longer chain short (17 tokens
-// 5.6).
+// ring, after they have read it. 8192 channels of a wider projection's rows, with the ring, us before (a
+// thread to an element, four loads each, and a launch for the ring) -> now: 17 tokens 4.2 -> 2.8, 717 tokens
+// 14.7 -> 7.6, 4096 tokens, 134 MB, 92 -> 32, 16384 tokens 352 -> 108.
+template <int V>
 __global__ __launch_bounds__(256) void conv_seq_kernel(const uint16_t* __restrict__ x, int ldx, int tokens,
                                                        int channels, const uint16_t* __restrict__ w,
                                                        uint16_t* __restrict__ ring, int pos0,
                                                        uint16_t* __restrict__ out, int ldo, int per) {
 #pragma clang fp contract(off)
-  const int c = blockIdx.x * 256 + threadIdx.x;
+  struct alignas(2 * V) Row {
+    uint16_t v[V];
+  };
+  const int c = (blockIdx.x * 256 + threadIdx.x) * V;
   if (c >= channels) return;
   const int t0 = blockIdx.y * per, t1 = min(t0 + per, tokens);
-  const uint2 wt = *reinterpret_cast<const uint2*>(w + (size_t)c * 4);
-  const float wk[4] = {__uint_as_float(wt.x << 16), __uint_as_float(wt.x & 0xFFFF0000u),
-                       __uint_as_float(wt.y << 16), __uint_as_float(wt.y & 0xFFFF0000u)};
-  auto load = [&](int t) { return bf2f(x[(size_t)t * ldx + c]); };
-  float h[7];  // rows t - 3 .. t + 3
+  float wk[V][4];
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    const uint2 wt = *reinterpret_cast<const uint2*>(w + (size_t)(c + v) * 4);
+    wk[v][0] = __uint_as_float(wt.x << 16), wk[v][1] = __uint_as_float(wt.x & 0xFFFF0000u);
+    wk[v][2] = __uint_as_float(wt.y << 16), wk[v][3] = __uint_as_float(wt.y & 0xFFFF0000u);
+  }
+  float h[V][7];  // rows t - 3 .. t + 3
+  auto load = [&](int t, int i) {
+    const Row r = *reinterpret_cast<const Row*>(x + (size_t)t * ldx + c);
+#pragma unroll
+    for (int v = 0; v < V; ++v) h[v][i] = bf2f(r.v[v]);
+  };
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     const int t = t0 - 3 + j;
-    h[j] = t >= 0 ? load(t) : bf2f(ring[(size_t)c * 4 + ((pos0 + t) & 3)]);
+    if (t >= 0) {
+      load(t, j);
+    } else {
+#pragma unroll
+      for (int v = 0; v < V; ++v) h[v][j] = bf2f(ring[(size_t)(c + v) * 4 + ((pos0 + t) & 3)]);
+    }
   }
   for (int t = t0; t < t1; t += 4) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) h[3 + i] = load(min(t + i, tokens - 1));
-    float s[4], y[4];
+    for (int i = 0; i < 4; ++i) load(min(t + i, tokens - 1), 3 + i);
+    Row o[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float acc = h[i] * wk[0];
-      acc = acc + h[i + 1] * wk[1];
-      acc = acc + h[i + 2] * wk[2];
-      acc = acc + h[i + 3] * wk[3];
-      s[i] = round_bf(acc);
+    for (int v = 0; v < V; ++v) {
+      float s[4], y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float acc = h[v][i] * wk[v][0];
+        acc = acc + h[v][i + 1] * wk[v][1];
+        acc = acc + h[v][i + 2] * wk[v][2];
+        acc = acc + h[v][i + 3] * wk[v][3];
+        s[i] = round_bf(acc);
+      }
+      silu_fast(s, y);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i].v[v] = f2bf(y[i]);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) h[v][j] = h[v][j + 4];
     }
-    silu_fast(s, y);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (t + i < t1) out[(size_t)(t + i) * ldo + c] = f2bf(y[i]);
-#pragma unroll
-    for (int j = 0; j < 3; ++j) h[j] = h[j + 4];
+      if (t + i < t1) *reinterpret_cast<Row*>(out + (size_t)(t + i) * ldo + c) = o[i];
   }
   if (t0 == 0) {
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       const int t = tokens - 3 + j;
-      if (t >= 0) ring[(size_t)c * 4 + ((pos0 + t) & 3)] = x[(size_t)t * ldx + c];
+      if (t < 0) continue;
+#pragma unroll
+      for (int v = 0; v < V; ++v) ring[(size_t)(c + v) * 4 + ((pos0 + t) & 3)] = x[(size_t)t * ldx + c + v];
     }
   }
 }
 
 // Tokens a thread walks: long walks read fewer rows twice, short ones fill the chip.
 static int conv_tokens(int tokens, int channels) { return (long)tokens * channels >= 1 << 23 ? 16 : 4; }
+// Channels to a thread: two make longer runs of memory, which long prompts are bound by (8192 channels, 4096
+// tokens 33.7 -> 31.7 us, 16384 118 -> 108; four are as fast), and a longer chain of ring accesses and
+// SiLUs, which short ones are (1024 tokens 11.6 -> 12.7; four: 17 tokens 2.8 -> 5.6).
+static bool conv_pairs(int tokens, int channels) { return (long)tokens * channels >= 1 << 24; }
 
 // ---------------------------------------------------------------------------------------
 // chunked gated delta rule (reference.py:403-461 over a sequence)
@@ -1523,8 +1551,12 @@ int df_causal_conv_prefill(const uint16_t* x, int ldx, int tokens, int channels,
       (reinterpret_cast<uintptr_t>(weight) & 7) || tokens > 65535)
     return DF_BAD_ARGUMENT;
   const int per = conv_tokens(tokens, channels);
-  hipLaunchKernelGGL(conv_seq_kernel, dim3((channels + 255) / 256, (tokens + per - 1) / per), dim3(256), 0, stream, x, ldx,
-                     tokens, channels, weight, ring, pos0, out, ldo, per);
+  const bool pairs = conv_pairs(tokens, channels) && channels % 2 == 0 && ldx % 2 == 0 && ldo % 2 == 0 &&
+                     !(reinterpret_cast<uintptr_t>(x) & 3) && !(reinterpret_cast<uintptr_t>(out) & 3);
+  const int width = pairs ? 512 : 256;  // channels a workgroup
+  hipLaunchKernelGGL(pairs ? conv_seq_kernel<2> : conv_seq_kernel<1>,
+                     dim3((channels + width - 1) / width, (tokens + per - 1) / per), dim3(256), 0, stream, x, ldx, tokens,
+                     channels, weight, ring, pos0, out, ldo, per);
   DF_RETURN_LAUNCH_STATUS();
 }
 

@@ -147,11 +147,11 @@ def test_causal_conv_prefill_is_conv1d(tokens, pos0):
 @pytest.mark.parametrize("tokens,pos0,channels,shift,pad", [
     (1, 2, 4, 0, 0), (3, 1, 1028, 0, 4), (4, 7, 1020, 0, 0), (5, 0, 6, 0, 2), (17, 3, 260, 4, 0), (17, 3, 260, 1, 0),
     (31, 6, 257, 0, 3), (2047, 5, 8, 0, 0), (2048, 0, 12, 0, 0), (2050, 9, 5, 0, 0), (1024, 2, 8191, 0, 1),
-    (1025, 3, 8192, 0, 0)])
+    (1025, 3, 8192, 0, 0), (2049, 3, 8194, 0, 0), (2049, 2, 8194, 1, 1)])
 def test_causal_conv_prefill_edges(tokens, pos0, channels, shift, pad):
     """Remainders of the tokens a thread walks (4 below 2^23 elements, 16 from there) and of a workgroup's
-    channels, rows that allow only 2-byte loads, and the history ring read and written by one call; exact,
-    as both sides take the taps in order in fp32."""
+    channels (two a thread from 2^24 elements), rows that allow only 2-byte loads, and the history ring read
+    and written by one call; exact, as both sides take the taps in order in fp32."""
     print(f"conv edges {tokens} {pos0} {channels} {shift} {pad}", flush=True)
     gen = torch.Generator().manual_seed(tokens + channels)
     rand = lambda *s: torch.randn(s, generator=gen).to(torch.bfloat16)
