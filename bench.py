@@ -72,7 +72,7 @@ GATE_UP_KERNEL = "w4_gemv_kernel<RMSNORM, SWIGLU> (post-attention norm + gate/up
 # over ``--roofline-only`` (12049 KiB fetched, 18 KiB written per launch), each scaled by what
 # the counter reads for a plain 256 MiB device copy (x 2.000 for FETCH_SIZE, x 1.000 for
 # WRITE_SIZE). Re-measure when the kernel changes.
-GATE_UP_TRAFFIC_BYTES = 12049 * 1024 * 2 + 18 * 1024
+GATE_UP_TRAFFIC_BYTES = 12030 * 1024 * 2 + 18 * 1024
 # HBM bytes per decode token of the persistent kernel from the calibrated PMC passes over the
 # timed 256-token launch (334,344,530.5 KiB fetched x 1.99982, 17,625,739.0 KiB written, / 256),
 # recorded with their commands in PERSISTENT_TRAFFIC_SOURCE. Re-measure when the kernel changes.

@@ -60,14 +60,14 @@ DF_DEVICE float readlane(float v, int lane) {
 //   products of this one; A operands are read a step (narrow shapes: more) ahead.
 // - WREG workgroups are persistent, one per CU: the next tile's first stage loads while the
 //   sums of this one meet in LDS, 32 rows at a time, and leave as 16-byte stores.
-// What bounds it: 128 x 256 tiles take 5950 cycles a stage for 4096 of products and 2200 of
-// dequant (MFMA and VALU of a SIMD's two waves share its issue), and with every CU busy the
-// clock falls to 1.73 GHz under the power limit (2.4 with 10 CUs busy). Before (128 x 128 tiles,
-// each wave all 128 rows x 32 columns on 16 x 16 x 32 products, x through registers, one
-// group's weights ahead) -> now, us: gate|up 4096 x 2560 x 18432 505 -> 360 (1074 TFLOP/s; a
-// plain bf16 library product of that shape 368), down 4096 x 9216 x 2560 301 -> 187, at 100
-// rows 38.6 -> 22.9 and 115 -> 26.5. Tried and not kept: 16 x 16 x 32 products (same stage time,
-// twice the operand reads), forcing products and VALU to alternate one by one (1 to 3 %
+// What bounds it: of a SIMD's cycles in the 4096 x 2560 x 18432 SwiGLU product (128 x 256 tiles) the matrix
+// cores are busy in 51 %, other VALU (mostly the dequant) takes 42 %, 23 % run both; waves wait for their turn
+// to issue 42 % of the time and for LDS, DMA and barriers 26 %. The clock averages 1.85 GHz of 2.4 there.
+// LDS hands out 36 bytes a cycle and CU. Before (128 x 128 tiles, each wave all 128 rows x 32
+// columns on 16 x 16 x 32 products, x through registers, one group's weights ahead) -> now, us: gate|up
+// 4096 x 2560 x 18432 433 -> 373 (1038 TFLOP/s; a plain bf16 library product of that shape 368), down 4096 x
+// 9216 x 2560 257 -> 201, at 100 rows 36.0 -> 23.5 and 104 -> 28.5. Tried and not kept: 16 x 16 x 32 products (same
+// time, twice the operand reads), forcing products and VALU to alternate one by one (1 to 3 %
 // slower), wave priorities (no change), 320-column tiles (spill).
 
 constexpr int kGmMaxLds = 160 * 1024;
@@ -788,7 +788,8 @@ DF_DEVICE void split3(float a, float b, uint32_t (&part)[3]) {
 //   3. every wave: S = e^gamma_C S + K^T delta (K read transposed by ds_read_tr16_b64), its planes.
 // Every operand that is a lane's own is loaded a chunk ahead into registers.
 // A serial chain of three steps a chunk, 2.5 us: 256 workgroups for 32 heads are one per CU, so
-// wider column tiles would idle CUs. Without any loads the loop takes about 95 of
+// wider column tiles would idle CUs. Waves wait 58 % of the time and the matrix cores are busy in 20 % of a
+// SIMD's cycles. Without any loads the loop takes about 95 of
 // the 157 us (4096 tokens, 32 heads), without T R too about 75. 319 us with the rows in fp32
 // and every product on the fp32 unit. The T, Q and V loads are issued after step 2's products:
 // at the start of step 1 they cost 12 us more, after its products 13.
@@ -955,7 +956,7 @@ __global__ __launch_bounds__(kScanThreads) void delta_scan_kernel(DfDeltaPrefill
       if (chunk + 1 < nchunks) issue_k(chunk + 1);
       const Outs mine = out;
       out = fetch_out(chunk);
-      if (chunk > 0) outputs(mine, chunk - 1);  // its stores last: nothing waits for them
+      if (chunk > 0) outputs(mine, chunk - 1);  // (the wait at the next chunk's top takes its stores in)
     }
     __syncthreads();
     // ---- 2: delta
@@ -1169,14 +1170,13 @@ __global__ __launch_bounds__(256) void qk_rows_kernel(DfQkPrefillArgs p, int per
 // does. A row's result depends only on its own scores in blocks of 32 keys from key 0, so a
 // prompt filled in chunks equals one pass.
 //
-// The next block's K products run between this block's softmax, so the VALU is hidden (without
-// it the kernel takes as long). What bounds it is LDS: per 64 keys a CU reads 256 KB of operands and
-// writes 64 KB, for 2048 cycles of products in about 4900 (without the DMA 20 % faster, without
-// either product 22 %). Causal prompts, us before (two passes over the keys, 16 query rows to a
-// wave) -> now: 8192 tokens 3106 -> 573 (959 TFLOP/s), 717 tokens 114 -> 38; 2000 tokens after
-// 20 000 keys 675 (1019 TFLOP/s). Measured and not kept: 64 positions to a workgroup and no key
-// sets (8192 tokens 562, 717 tokens 55), two barriers with K and V two blocks ahead (595),
-// reading an operand right before its product (597).
+// The next block's K products run between this block's softmax. No unit is full (8192 tokens): of a SIMD's
+// cycles the matrix cores are busy in 41 %, other VALU takes 29 %, 15 % run both, LDS hands out 53 bytes a
+// cycle and CU; waves wait for LDS, DMA and barriers 39 % of the time and for their turn to issue 27 %.
+// Causal prompts, us before (two passes over the keys, 16 query rows to a wave) -> now: 8192
+// tokens 3106 -> 573 (959 TFLOP/s), 717 tokens 114 -> 38; 2000 tokens after 20 000 keys 675 (1019 TFLOP/s).
+// Measured and not kept: 64 positions to a workgroup and no key sets (8192 tokens 562, 717 tokens 55), two
+// barriers with K and V two blocks ahead (595), reading an operand right before its product (597).
 
 constexpr int kAtKeys = 64;
 constexpr int kAtTile = kAtKeys * kHd * 2;  // bytes of a K or V block
@@ -1486,14 +1486,14 @@ static hipError_t launch_gemm_shape(const DfInt4GemmArgs& a, hipStream_t stream)
   return hipGetLastError();
 }
 
-// The shapes, and the cost of one workgroup in each: start and epilogue, and a stage (ns). Fitted
-// to 60 measured (M, K, N): the four projections of the model at 17 .. 8192 rows. A launch
+// The shapes, and the cost of one workgroup in each: start and epilogue, and a stage (ns). A launch
 // takes as many rounds of one workgroup per CU as it has tiles, so the shape taken is the one
-// with the least rounds * (start + stages * stage); over the 60 it was the fastest of the
-// seven but for 0.04 %. Wide ones serve long prompts (2560 x 18432 at 4096 rows: 9 full rounds of
-// 128 x 256, 360 us against 410 with 128 x 128), 96 rows where they pack better (9216 x 2560 at
-// 4096 rows: 187 us against 222), narrow ones reach more CUs with a short prompt (9216 x 2560
-// at 100 rows: 26.5 us with 32 x 64 against 96 with 128 x 256).
+// with the least rounds * (start + stages * stage). Of 65 products (the model's five projections at 17 ..
+// 8192 rows, all seven shapes timed) it is the fastest in 64 and 0.6 % slower than that in one. As a time
+// the cost is up to 15 % low where the clock falls (320 us for 376), alike for the wide shapes. Wide ones serve
+// long prompts (2560 x 18432 at 4096 rows: 9 full rounds of 128 x 256, 376 us against 443 with 128 x 128), 96
+// rows where they pack better (9216 x 2560 at 4096 rows: 197 us against 229), narrow ones reach more CUs
+// with a short prompt (9216 x 2560 at 100 rows: 27.3 us with 32 x 64 against 97 with 128 x 256).
 struct GemmCost {
   int bm, bn, start, stage;
 };
@@ -1538,7 +1538,7 @@ int df_int4_gemm(const DfInt4GemmArgs* a, hipStream_t stream) {
   const int out_cols = a->epilogue == DF_EPI_SWIGLU ? a->N / 2 : a->N;
   if (a->ldx < a->K || a->ldx % 8 || a->ldo < out_cols || !aligned16(a->x) || !aligned16(a->w))
     return DF_BAD_ARGUMENT;
-  // row blocks of the smallest shape fit the grid
+  // (8.4 M rows: tile and row counts stay far inside int)
   if ((a->M + 127) / 128 > 65535) return DF_BAD_ARGUMENT;
   const int shape = gemm_plan(a->M, a->K, a->N);
   const hipError_t e = a->epilogue == DF_EPI_SWIGLU ? launch_gemm<DF_EPI_SWIGLU>(*a, shape, stream)

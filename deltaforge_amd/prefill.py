@@ -17,8 +17,10 @@ Then RMSNorm, the tied head and the argmax of the last position.
 ``Prefiller.fill(decoder, prompt)`` leaves a ``PersistentDecoder`` (``fill_engine`` a
 ``DecodeEngine``, one sequence per row) in the state its own token-by-token prefill would:
 the conv rings, recurrent states and KV caches of every layer, the position, the last logits
-and the first generated token. Summation order is the only difference. ``Prefiller`` keeps its own copy of the weights, in natural column order (the
-persistent kernel's copy is permuted XCD-major).
+and the first generated token. The differences are the order of fp32 sums and, in attention from the
+33rd position on, probabilities rounded to bf16 before their division by the sum. ``Prefiller``
+keeps its own copy of the weights, in natural column order (the persistent kernel's copy is
+permuted XCD-major).
 """
 
 from __future__ import annotations

@@ -260,8 +260,8 @@ int df_argmax(const uint16_t* logits, int rows, int n, int64_t* tokens, int64_t*
  * The reference runs a prompt through ReferenceModel.forward with seq_len = P
  * (reference.py:779-817): the projections as [P, K] x [K, N] products, the conv over the
  * sequence, the sequential delta-rule scan (reference.py:450-458) and causal attention. These
- * entry points are that forward's pieces. Rounding points are the reference's; only fp32
- * summation order differs. */
+ * entry points are that forward's pieces. Rounding points are the reference's but for one, in
+ * df_attention_prefill; otherwise only fp32 summation order differs. */
 
 /* out = bf16(x @ bf16(dequant(W))), fp32 sums, W in the device tiling of df_int4_repack
  * (reference kernels/quantised_linear.py GEMV_MAX_ROWS dense fallback, which dequantises and
@@ -333,10 +333,11 @@ typedef struct DfQkPrefillArgs {
 int df_qk_norm_rope_prefill(const DfQkPrefillArgs* args, hipStream_t stream);
 
 /* Causal GQA attention of `tokens` queries at positions pos0 .. over cache rows 0 .. pos
- * (reference.py:645-677): scores = bf16(bf16(q.k) * scale), p = bf16(softmax_fp32),
- * o = bf16(p V), out = bf16(o * bf16(gate_fn(gate))) with gate_fn sigmoid (gate_kind 0) or
- * silu (1). Hq = 4 Hkv, head_dim 256. gate of head h, token t: gate[t * ld_gate + h *
- * gate_head_stride + d]. */
+ * (reference.py:645-677): scores = bf16(bf16(q.k) * scale) for any scale, p = softmax_fp32,
+ * o = bf16(bf16(p) V) at positions below 32 and, with the same relative rounding, o = bf16(bf16(e) V /
+ * sum e), e = exp(score - m) for a running maximum m, from there on, out = bf16(o *
+ * bf16(gate_fn(gate))) with gate_fn sigmoid (gate_kind 0) or silu (1). Hq = 4 Hkv, head_dim 256. gate
+ * of head h, token t: gate[t * ld_gate + h * gate_head_stride + d]. */
 typedef struct DfAttnPrefillArgs {
   const uint16_t* q;
   const uint16_t* k_cache;
