@@ -69,7 +69,7 @@ def log(msg: str) -> None:
 
 GATE_UP_KERNEL = "w4_gemv_kernel<RMSNORM, SWIGLU> (post-attention norm + gate/up 2560 x 18432 + SwiGLU)"
 # HBM bytes one gate/up launch actually moves: rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE passes
-# over ``--roofline-only`` (12049 KiB fetched, 18 KiB written per launch), each scaled by what
+# over ``--roofline-only`` (12030 KiB fetched, 18 KiB written per launch), each scaled by what
 # the counter reads for a plain 256 MiB device copy (x 2.000 for FETCH_SIZE, x 1.000 for
 # WRITE_SIZE). Re-measure when the kernel changes.
 GATE_UP_TRAFFIC_BYTES = 12030 * 1024 * 2 + 18 * 1024
