@@ -157,7 +157,8 @@ DF_DEVICE void silu_bits(const float (&x)[N], float (&y)[N]) {
     const float d = 1.0f + ldexpf(__builtin_amdgcn_exp2f(f), static_cast<int>(n));
     const float r0 = __builtin_amdgcn_rcpf(d), r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
     const float q = x[i] * r;
-    y[i] = copysignf(fmaf(fmaf(-d, q, x[i]), r, q), x[i]);  // (-0 stays so)
+    const float quot = copysignf(fmaf(fmaf(-d, q, x[i]), r, q), x[i]);  // (-0 stays so)
+    y[i] = x[i] > 104.0f ? x[i] : quot;                                 // (and +inf)
     low = fminf(low, x[i]);
   }
   if (__builtin_expect(low < -80.0f, 0)) {

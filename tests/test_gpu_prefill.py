@@ -309,11 +309,11 @@ def test_gated_rms_norm_rows_edges(tokens, heads, shift, pad):
 def test_gated_rms_norm_rows_gate_is_fp32():
     """The gate's SiLU goes into the product unrounded, so results are compared with the product in 64
     bits, rounded once. x is +-1 and eps 0, so that the norm is x itself; a head has one z, all of a
-    weight's mantissas. z is every bf16 from -80 to 104. The gate is off by 3 x 2^-23 at most (2 for e^-z,
+    weight's mantissas. z is every bf16 from -80 to 1e38. The gate is off by 3 x 2^-23 at most (2 for e^-z,
     half for 1 + e^-z, half for the quotient), the product by 2^-24: a result may round the other way only
     that near to the middle of two bf16."""
     bits = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
-    z = bits[(bits.float() >= -80) & (bits.float() <= 104) & (bits.float().abs() > 1e-30)]
+    z = bits[(bits.float() >= -80) & (bits.float() <= 1e38) & (bits.float().abs() > 1e-30)]
     z = torch.cat([z, z[:-z.numel() % 32]]).reshape(-1, 32, 1).expand(-1, 32, 128).reshape(-1, 32 * 128)
     x = torch.where(torch.arange(z.shape[1]) % 3 == 0, -1.0, 1.0).to(torch.bfloat16).expand(z.shape).contiguous()
     w = (1 + torch.arange(128) / 128).to(torch.bfloat16)
@@ -324,6 +324,17 @@ def test_gated_rms_norm_rows_gate_is_fp32():
     spacing = 2.0 ** (torch.floor(torch.log2(want.abs())) - 7)  # of bf16 at want
     wrong = off > 0.5 * spacing + 3.5 * 2.0**-23 * want.abs()
     assert not wrong.any(), f"{int(wrong.sum())} results, z from {float(z[wrong].min())} to {float(z[wrong].max())}"
+
+
+def test_gated_rms_norm_rows_gate_of_zeros_infinities_and_nan():
+    """Each element's own: SiLU keeps a zero's sign and +inf, and has no value at -inf (0 times inf)."""
+    inf, nan = float("inf"), float("nan")
+    z = torch.tensor([0.0, -0.0, inf, -inf, nan, 3e38, -3e38, 1.0], dtype=torch.bfloat16).repeat(16).reshape(1, 128)
+    ones = torch.ones((1, 128), dtype=torch.bfloat16, device=DEV)
+    got = gated_rms_norm_rows(ones, z.to(DEV), ones[0].contiguous(), 0.0).cpu().float()[0, :8]
+    assert got[0] == 0 and got[1] == 0 and torch.signbit(got[:2]).tolist() == [False, True]
+    assert got[2] == inf and torch.isnan(got[3:5]).all()
+    assert got[5] == z[0, 5].float() and abs(got[6]) < 2e-37 and got[7] == torch.tensor(0.7310586).bfloat16().float()
 
 
 @pytest.mark.parametrize("tokens,hq,hkv,half,pos0,shift", [
